@@ -145,6 +145,7 @@ def measure_case(label, ins, outs, rank, dtype_name, init, tokens, steps, warmup
         max_ref = ref.abs().max().item()
         del y, yf, ref, diff
         info = run.selected(T)
+        flops = m.launch_flops(info, spec, T)
         ref_flops = m.reference_flops(spec, T)
         peak = m.PEAK_TFLOPS[dtype]
         case = {
@@ -154,14 +155,14 @@ def measure_case(label, ins, outs, rank, dtype_name, init, tokens, steps, warmup
             "ours_stream_us": ours_us, "dense_stream_us": dense_us,
             "speedup_vs_dense": dense_us / ours_us,
             "ours_host_us": host_ours, "dense_host_us": host_dense, "ours_submit_us": submit_us,
-            "flops": info["flops"], "bytes": info["bytes"],
+            "flops": flops, "bytes": info["bytes"],
             "max_abs_err_vs_fp32": err, "max_abs_ref": max_ref,
             "prepare_ms": prep_ms, "packed_bytes": run.packed_bytes,
             "prepare_held_bytes": prep_held, "prepare_peak_bytes": prep_peak,
             "call_extra_bytes": call_extra,
             "dense_weight_bytes": weight.numel() * weight.element_size(),
             "passed": ok,
-            **m.roofline(info["flops"], info["bytes"], ours_us, dtype),
+            **m.roofline(flops, info["bytes"], ours_us, dtype),
             # the reference's flop count (its fixed order) at the same time, for comparison
             # with its "% FP16 TC peak" column
             "reference_flops": ref_flops,

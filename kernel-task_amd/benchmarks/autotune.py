@@ -189,7 +189,10 @@ def tune_shape(shape: tilegen.ShapeDecl, budget_s: float,
     for r in ranges:
         r["order"] = list(tiles[r["name"]][0])
         r["tile"] = asdict(tiles[r["name"]][1])
-    return ({"order": list(order), "device": torch.cuda.get_device_name(0), "ranges": ranges},
+    joined = [r for r in ranges if r["tile"]["JN"]]
+    return ({"order": list(order), "device": torch.cuda.get_device_name(0),
+             "ranges": [r for r in ranges if not r["tile"]["JN"]],
+             **({"joined": joined} if joined else {})},
             {str(T): row for T, row in measured.items()})
 
 

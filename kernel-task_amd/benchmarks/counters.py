@@ -48,7 +48,7 @@ def _rows(run_dir: Path) -> list[dict]:
 def kernel_label(name: str) -> str | None:
     """'ring3<KCfg fields>' for a tensor-ring kernel, 'copy' for the runtime's buffer copy,
     None for anything else (allocation fills, packing, random inputs)."""
-    if "ring3_mfma" in name:
+    if "ring3_mfma" in name or "ring3_join_kernel" in name:
         m = re.search(r"KCfg\{([^}]*)\}", name)
         return "ring3<" + (m.group(1).replace(" ", "") if m else "?") + ">"
     if "ring3_generic" in name:
@@ -178,14 +178,14 @@ def grids(trace: Path, max_gap_us: float = 30.0) -> list[dict]:
 
 
 def kcfg_of(label: str) -> tuple[tuple, tuple] | None:
-    """(chain order, tile fields TT..TP) of a 'ring3<KCfg fields>' label; fields the
-    compiler's name leaves out at the end are zero."""
+    """(chain order, tile fields TT..TP, and JN for joined-core tiles) of a 'ring3<KCfg fields>'
+    label; fields the compiler's name leaves out at the end are zero."""
     m = re.fullmatch(r"ring3<([-0-9,]*)>", label)
     if not m:
         return None
     f = [int(v) for v in m.group(1).split(",") if v]
-    f += [0] * (27 - len(f))
-    return tuple(f[1:4]), tuple(f[11:27])
+    f += [0] * (28 - len(f))
+    return tuple(f[1:4]), tuple(f[11:28 if f[27] else 27])
 
 
 def cases(trace: Path, details: dict, max_gap_us: float = 30.0) -> list[dict]:
@@ -207,7 +207,8 @@ def cases(trace: Path, details: dict, max_gap_us: float = 30.0) -> list[dict]:
     out = []
     for c in details["cases"]:
         order, tile = tilegen.parse_variant_name(c["variant"])
-        key = ((tuple(order), dataclasses.astuple(tile)), tuple(c["grid"][:2]))
+        fields = dataclasses.astuple(tile)
+        key = ((tuple(order), fields if tile.JN else fields[:-1]), tuple(c["grid"][:2]))
         r = by_cfg.get(key)
         row = {"case": c["case"], "tokens": c["tokens"], "variant": c["variant"],
                "grid": c["grid"][:2], "stream_us": c["ours_stream_us"]}

@@ -68,6 +68,10 @@ def run(form: str, tokens: int, layers: list[int], timeout: float = 240.0,
     path = binary(form)
     if not path.exists():
         raise RuntimeError(f"{path} is not built; run with --build first")
+    # the program reads the library's plans through the headers it was compiled with: one from
+    # before a change to them would take its device pointers from the wrong fields
+    if path.stat().st_mtime < build_ext._newest_dependency():
+        raise RuntimeError(f"{path} is older than the headers of libtrk.so; run with --build first")
     env = dict(os.environ)
     if parallel:
         env["STACK_PAR"] = str(parallel)

@@ -12,7 +12,6 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape012, 1, 1, 8, 32, 4, 2, 1, 4, 32, 8), 2, 4)  // wide4x32w8_t1k2n1_ic4
     TRK_ENTRY(tile(kShape012, 1, 1, 12, 32, 4, 2, 1, 8, 32, 8), 5, 8)  // wide8x32w8_t1k2n1_ic4
     TRK_ENTRY(tile(kShape012, 2, 1, 12, 32, 2, 1, 2, 8, 32, 8, 1), 9, 16)  // wide8x32w8_t2k1n2_p
-    TRK_ENTRY(tile(kShape012, 4, 1, 12, 32, 2, 1, 2, 8, 32, 8), 17, 1073741824)  // wide8x32w8_t4k1n2
 };
 
 }  // namespace

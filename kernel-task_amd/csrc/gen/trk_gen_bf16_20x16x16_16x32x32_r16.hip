@@ -11,7 +11,7 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape012, 1, 1, 4, 16, 4, 8, 1, 0, 16, 8), 1, 1)  // t1_l16_s4_w8_k8
     TRK_ENTRY(tile(kShape012, 1, 1, 8, 32, 4, 2, 1, 4, 32, 8), 2, 4)  // wide4x32w8_t1k2n1_ic4
     TRK_ENTRY(tile(kShape012, 1, 1, 16, 32, 2, 2, 1, 8, 32, 8, 2), 5, 8)  // wide8x32w8_t1k2n1_ic2_p2
-    TRK_ENTRY(tile(kShape012, 1, 2, 16, 32, 2, 1, 2, 8, 32, 8, 1), 9, 1073741824)  // wide8x32w8_f2k1n2_ic2_p
+    TRK_ENTRY(tile(kShape012, 1, 2, 16, 32, 2, 1, 2, 8, 32, 8, 1), 9, 32)  // wide8x32w8_f2k1n2_ic2_p
 };
 
 }  // namespace

@@ -12,9 +12,6 @@ const Entry kEntries[] = {
     TRK_ENTRY_PAIR(tile(kShape021, 1, 1, 16, 34, 2, 2, 1, 8, 32, 8, 1), 2, 8)  // wide8x32w8_t1k2n1_ic2_p
     TRK_ENTRY_PAIR(tile(kShape021, 1, 2, 16, 34, 2, 1, 2, 8, 32, 8), 9, 16)  // wide8x32w8_f2k1n2_ic2
     TRK_ENTRY_PAIR(tile(kShape021, 4, 1, 16, 34, 1, 1, 2, 8, 32, 8, 1), 17, 32)  // wide8x32w8_t4k1n2_p
-    TRK_ENTRY_PAIR(tile(kShape021, 1, 2, 16, 34, 2, 1, 2, 8, 32, 8), 33, 64)  // wide8x32w8_f2k1n2_ic2
-    TRK_ENTRY_PAIR(tile(kShape021, 4, 1, 16, 34, 1, 1, 2, 8, 32, 8, 1), 65, 128)  // wide8x32w8_t4k1n2_p
-    TRK_ENTRY_PAIR(tile(kShape021, 1, 2, 16, 34, 2, 1, 2, 8, 32, 8), 129, 1073741824)  // wide8x32w8_f2k1n2_ic2
 };
 
 }  // namespace

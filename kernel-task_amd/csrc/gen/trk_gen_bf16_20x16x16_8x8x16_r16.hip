@@ -14,7 +14,6 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape012, 1, 1, 2, 16, 4, 4, 1), 5, 8)  // t1_s2
     TRK_ENTRY(tile(kShape012, 1, 1, 8, 16, 4, 2, 1, 8, 32, 8, 1), 9, 32)  // wide8x32w8_t1k2n1_ic4_p
     TRK_ENTRY(tile(kShape012, 1, 2, 8, 16, 4, 1, 2, 8, 32, 8), 33, 64)  // wide8x32w8_f2k1n2_ic4
-    TRK_ENTRY(tile(kShape012, 4, 1, 8, 16, 2, 2, 1, 8, 32, 8, 1), 65, 1073741824)  // wide8x32w8_p
 };
 
 }  // namespace

@@ -12,7 +12,7 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape012, 1, 1, 4, 10, 4, 4, 1), 2, 2)  // t1_l10_s4_k4
     TRK_ENTRY(tile(kShape012, 1, 1, 8, 20, 4, 2, 1, 4, 32, 8), 3, 8)  // wide4x32w8_t1k2n1_ic4
     TRK_ENTRY(tile(kShape012, 1, 1, 16, 20, 4, 2, 1, 8, 32, 8), 9, 16)  // wide8x32w8_t1k2n1_ic4
-    TRK_ENTRY(tile(kShape012, 1, 2, 16, 20, 2, 1, 2, 8, 32, 8, 1), 17, 1073741824)  // wide8x32w8_f2k1n2_ic2_p
+    TRK_ENTRY(tile(kShape012, 1, 2, 16, 20, 2, 1, 2, 8, 32, 8, 1), 17, 32)  // wide8x32w8_f2k1n2_ic2_p
 };
 
 }  // namespace

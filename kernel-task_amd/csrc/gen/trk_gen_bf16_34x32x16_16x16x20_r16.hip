@@ -11,8 +11,7 @@ constexpr Shape kShape102{TRK_DTYPE_BF16, 1, 0, 2, 34, 32, 16, 16, 16, 20, 16};
 const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape012, 1, 1, 2, 10, 2, 8, 1, 0, 16, 8), 1, 1)  // t1_l10_s2_w8_k8
     TRK_ENTRY(tile(kShape012, 1, 1, 4, 10, 1, 8, 1, 0, 16, 8, 1), 2, 2)  // t1_l10_s4_w8_k8_p
-    TRK_ENTRY(tile(kShape102, 1, 1, 4, 20, 1, 2, 2), 3, 16)  // mid_1of4_k2@102
-    TRK_ENTRY(tile(kShape012, 4, 1, 8, 20, 1, 2, 1, 4, 32, 4), 17, 1073741824)  // wide4x32_relaxed
+    TRK_ENTRY(tile(kShape102, 1, 1, 4, 20, 1, 2, 2), 3, 8)  // mid_1of4_k2@102
 };
 
 }  // namespace

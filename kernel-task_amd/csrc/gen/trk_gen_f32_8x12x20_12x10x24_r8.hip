@@ -15,7 +15,7 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape210, 1, 2, 10, 12, 4, 4, 1, 8, 32, 8, 1), 9, 16)  // ring3_mfma_wide8x32w8p<210,1,2,10,12,4,4,1>
     TRK_ENTRY(tile(kShape210, 1, 3, 10, 12, 4, 4, 1, 8, 32, 8), 17, 32)  // wide8x32w8_f3k4n1_ic4
     TRK_ENTRY(tile(kShape210, 1, 6, 10, 12, 2, 2, 1, 8, 32, 8, 1), 33, 64)  // wide8x32w8_f6k2n1_ic2_p
-    TRK_ENTRY(tile(kShape102, 1, 2, 12, 24, 2, 1, 2, 4, 32, 4), 65, 1073741824)  // ring3_mfma_wide4x32<102,1,2,12,24,2,1,2>
+    TRK_ENTRY(tile(kShape102, 1, 2, 12, 24, 2, 1, 2, 4, 32, 4), 65, 80)  // ring3_mfma_wide4x32<102,1,2,12,24,2,1,2>
     TRK_ENTRY(tile(kShape210, 2, 3, 10, 12, 1, 2, 1, 8, 32, 8, 1), 0, 0)  // cover_t2f3_p
 };
 

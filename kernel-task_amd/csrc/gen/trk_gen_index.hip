@@ -21,6 +21,22 @@ int mfma_register_gen_bf16_24x16x16_16x16x20_r8(Plan *plan);
 int mfma_register_gen_bf16_24x16x16_16x16x20_r16(Plan *plan);
 int mfma_register_gen_bf16_20x16x16_16x32x32_r8(Plan *plan);
 int mfma_register_gen_bf16_20x16x16_16x32x32_r16(Plan *plan);
+int join_register_gen_f16_8x12x20_12x10x24_r8(Plan *plan);
+int join_register_gen_f16_8x12x20_12x10x24_r16(Plan *plan);
+int join_register_gen_bf16_16x16x16_16x28x32_r8(Plan *plan);
+int join_register_gen_bf16_16x28x32_16x16x16_r16(Plan *plan);
+int join_register_gen_f32_8x12x20_12x10x24_r8(Plan *plan);
+int join_register_gen_bf16_20x16x16_16x34x32_r8(Plan *plan);
+int join_register_gen_bf16_20x16x16_16x34x32_r16(Plan *plan);
+int join_register_gen_bf16_34x32x16_16x16x20_r8(Plan *plan);
+int join_register_gen_bf16_34x32x16_16x16x20_r16(Plan *plan);
+int join_register_gen_bf16_20x16x16_16x24x32_r8(Plan *plan);
+int join_register_gen_bf16_20x16x16_16x24x32_r16(Plan *plan);
+int join_register_gen_bf16_20x16x16_8x8x16_r8(Plan *plan);
+int join_register_gen_bf16_20x16x16_8x8x16_r16(Plan *plan);
+int join_register_gen_bf16_24x16x16_16x16x20_r8(Plan *plan);
+int join_register_gen_bf16_24x16x16_16x16x20_r16(Plan *plan);
+int join_register_gen_bf16_20x16x16_16x32x32_r16(Plan *plan);
 
 int mfma_register_generated(Plan *plan) {
     int added = 0;
@@ -41,6 +57,22 @@ int mfma_register_generated(Plan *plan) {
     added += mfma_register_gen_bf16_24x16x16_16x16x20_r16(plan);
     added += mfma_register_gen_bf16_20x16x16_16x32x32_r8(plan);
     added += mfma_register_gen_bf16_20x16x16_16x32x32_r16(plan);
+    added += join_register_gen_f16_8x12x20_12x10x24_r8(plan);
+    added += join_register_gen_f16_8x12x20_12x10x24_r16(plan);
+    added += join_register_gen_bf16_16x16x16_16x28x32_r8(plan);
+    added += join_register_gen_bf16_16x28x32_16x16x16_r16(plan);
+    added += join_register_gen_f32_8x12x20_12x10x24_r8(plan);
+    added += join_register_gen_bf16_20x16x16_16x34x32_r8(plan);
+    added += join_register_gen_bf16_20x16x16_16x34x32_r16(plan);
+    added += join_register_gen_bf16_34x32x16_16x16x20_r8(plan);
+    added += join_register_gen_bf16_34x32x16_16x16x20_r16(plan);
+    added += join_register_gen_bf16_20x16x16_16x24x32_r8(plan);
+    added += join_register_gen_bf16_20x16x16_16x24x32_r16(plan);
+    added += join_register_gen_bf16_20x16x16_8x8x16_r8(plan);
+    added += join_register_gen_bf16_20x16x16_8x8x16_r16(plan);
+    added += join_register_gen_bf16_24x16x16_16x16x20_r8(plan);
+    added += join_register_gen_bf16_24x16x16_16x16x20_r16(plan);
+    added += join_register_gen_bf16_20x16x16_16x32x32_r16(plan);
     return added;
 }
 

@@ -1,0 +1,25 @@
+// Generated by kernel-task_amd/factorized_inference/tilegen.py; do not edit.
+// qwen_attn_q_gate: (20,16,16) -> (16,24,32), rank 8, bf16, chain order (1,2,0); token ranges measured by kernel-task_amd/benchmarks/autotune.py.
+#include "trk_join_kernel.h"
+
+namespace trk {
+namespace {
+
+constexpr Shape kShape120{TRK_DTYPE_BF16, 1, 2, 0, 20, 16, 16, 16, 24, 32, 8};
+
+const Entry kEntries[] = {
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 513, 640)  // ring3_join<120,128,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN(tile(kShape120, 160, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 641, 768)  // ring3_join<120,160,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 769, 1024)  // ring3_join<120,128,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN(tile(kShape120, 160, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1025, 1536)  // ring3_join<120,160,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1537, 3072)  // ring3_join<120,128,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN(tile(kShape120, 160, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 3073, 1073741824)  // ring3_join<120,160,1,8,16,1,1,2>
+};
+
+}  // namespace
+
+int join_register_gen_bf16_20x16x16_16x24x32_r8(Plan *plan) {
+    return register_entries(plan, kEntries, int(sizeof(kEntries) / sizeof(kEntries[0])));
+}
+
+}  // namespace trk

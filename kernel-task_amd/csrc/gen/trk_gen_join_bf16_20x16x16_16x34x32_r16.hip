@@ -1,0 +1,30 @@
+// Generated by kernel-task_amd/factorized_inference/tilegen.py; do not edit.
+// qwen_mlp_gate_up: (20,16,16) -> (16,34,32), rank 16, bf16, chain order (1,2,0); token ranges measured by kernel-task_amd/benchmarks/autotune.py.
+#include "trk_join_kernel.h"
+
+namespace trk {
+namespace {
+
+constexpr Shape kShape120{TRK_DTYPE_BF16, 1, 2, 0, 20, 16, 16, 16, 34, 32, 16};
+
+const Entry kEntries[] = {
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 48, 3, 1, 16, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 33, 48)  // ring3_join<120,48,3,1,16,1,4,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 64, 3, 1, 16, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 49, 64)  // ring3_join<120,64,3,1,16,1,4,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 80, 1, 1, 16, 1, 4, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 65, 80)  // ring3_join<120,80,1,1,16,1,4,2>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 128, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 81, 128)  // ring3_join<120,128,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 192, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 129, 192)  // ring3_join<120,192,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 193, 256)  // ring3_join<120,256,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 128, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 257, 384)  // ring3_join<120,128,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 192, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 385, 512)  // ring3_join<120,192,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 513, 768)  // ring3_join<120,256,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 192, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 769, 896)  // ring3_join<120,192,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 897, 1073741824)  // ring3_join<120,256,1,8,16,1,1,1>
+};
+
+}  // namespace
+
+int join_register_gen_bf16_20x16x16_16x34x32_r16(Plan *plan) {
+    return register_entries(plan, kEntries, int(sizeof(kEntries) / sizeof(kEntries[0])));
+}
+
+}  // namespace trk

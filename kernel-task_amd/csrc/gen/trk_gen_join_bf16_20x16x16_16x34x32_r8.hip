@@ -1,0 +1,32 @@
+// Generated by kernel-task_amd/factorized_inference/tilegen.py; do not edit.
+// qwen_mlp_gate_up: (20,16,16) -> (16,34,32), rank 8, bf16, chain order (1,2,0); token ranges measured by kernel-task_amd/benchmarks/autotune.py.
+#include "trk_join_kernel.h"
+
+namespace trk {
+namespace {
+
+constexpr Shape kShape120{TRK_DTYPE_BF16, 1, 2, 0, 20, 16, 16, 16, 34, 32, 8};
+
+const Entry kEntries[] = {
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 64, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 161, 192)  // ring3_join<120,64,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 96, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 225, 256)  // ring3_join<120,96,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 112, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 257, 320)  // ring3_join<120,112,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 128, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 321, 384)  // ring3_join<120,128,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 160, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 385, 448)  // ring3_join<120,160,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 192, 2, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 449, 512)  // ring3_join<120,192,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 128, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 513, 640)  // ring3_join<120,128,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 160, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 641, 1024)  // ring3_join<120,160,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 192, 2, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1025, 1280)  // ring3_join<120,192,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 128, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1281, 1536)  // ring3_join<120,128,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 192, 2, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1537, 2048)  // ring3_join<120,192,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 128, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 2049, 3072)  // ring3_join<120,128,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 160, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 3073, 1073741824)  // ring3_join<120,160,1,8,16,1,1,2>
+};
+
+}  // namespace
+
+int join_register_gen_bf16_20x16x16_16x34x32_r8(Plan *plan) {
+    return register_entries(plan, kEntries, int(sizeof(kEntries) / sizeof(kEntries[0])));
+}
+
+}  // namespace trk

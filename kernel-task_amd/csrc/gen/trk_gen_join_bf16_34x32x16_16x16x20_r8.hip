@@ -1,0 +1,22 @@
+// Generated by kernel-task_amd/factorized_inference/tilegen.py; do not edit.
+// qwen_mlp_down: (34,32,16) -> (16,16,20), rank 8, bf16, chain order (1,2,0); token ranges measured by kernel-task_amd/benchmarks/autotune.py.
+#include "trk_join_kernel.h"
+
+namespace trk {
+namespace {
+
+constexpr Shape kShape120{TRK_DTYPE_BF16, 1, 2, 0, 34, 32, 16, 16, 16, 20, 8};
+
+const Entry kEntries[] = {
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 4, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 641, 768)  // ring3_join<120,128,2,4,16,1,1,2>
+    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 4, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 769, 1024)  // ring3_join<120,192,2,4,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 4, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1025, 1073741824)  // ring3_join<120,128,2,4,16,1,1,2>
+};
+
+}  // namespace
+
+int join_register_gen_bf16_34x32x16_16x16x20_r8(Plan *plan) {
+    return register_entries(plan, kEntries, int(sizeof(kEntries) / sizeof(kEntries[0])));
+}
+
+}  // namespace trk

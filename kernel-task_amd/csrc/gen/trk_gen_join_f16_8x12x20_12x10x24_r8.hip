@@ -1,0 +1,27 @@
+// Generated by kernel-task_amd/factorized_inference/tilegen.py; do not edit.
+// r8: (8,12,20) -> (12,10,24), rank 8, f16, chain order (1,2,0); token ranges measured by kernel-task_amd/benchmarks/autotune.py.
+#include "trk_join_kernel.h"
+
+namespace trk {
+namespace {
+
+constexpr Shape kShape120{TRK_DTYPE_F16, 1, 2, 0, 8, 12, 20, 12, 10, 24, 8};
+
+const Entry kEntries[] = {
+    TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 4, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 161, 256)  // ring3_join<120,64,1,4,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 64, 2, 1, 12, 1, 4, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 257, 320)  // ring3_join<120,64,2,1,12,1,4,2>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 321, 512)  // ring3_join<120,128,1,4,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 8, 12, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 513, 768)  // ring3_join<120,96,1,8,12,1,1,2>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 12, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 769, 1024)  // ring3_join<120,128,1,8,12,1,1,2>
+    TRK_ENTRY_JOIN(tile(kShape120, 160, 1, 8, 12, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1025, 1280)  // ring3_join<120,160,1,8,12,1,1,2>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 8, 12, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1281, 1536)  // ring3_join<120,96,1,8,12,1,1,2>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 12, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1537, 1073741824)  // ring3_join<120,128,1,8,12,1,1,2>
+};
+
+}  // namespace
+
+int join_register_gen_f16_8x12x20_12x10x24_r8(Plan *plan) {
+    return register_entries(plan, kEntries, int(sizeof(kEntries) / sizeof(kEntries[0])));
+}
+
+}  // namespace trk

@@ -58,7 +58,7 @@ int plan_chain(Plan *p, const int order[3], int sg, int lg, int sfrag) {
     auto same_order = [&](const Chain &c) { return std::equal(order, order + 3, c.order); };
     for (int i = 0; i < p->nchains; ++i) {
         const Chain &o = p->chains[i];
-        if (same_order(o) && o.sg == sg && o.lg == lg && o.sfrag == sfrag) return i;
+        if (!o.join && same_order(o) && o.sg == sg && o.lg == lg && o.sfrag == sfrag) return i;
     }
     if (p->nchains == kMaxChains) return -1;
     Chain &c = p->chains[p->nchains];
@@ -66,11 +66,12 @@ int plan_chain(Plan *p, const int order[3], int sg, int lg, int sfrag) {
     c.sg = sg;
     c.lg = lg;
     c.sfrag = sfrag;
+    c.join = 0;
     c.ownF = c.ownS = c.ownL = 1;
     // sections whose layout an earlier chain of this order already has are shared
     for (int i = 0; i < p->nchains; ++i) {
         const Chain &o = p->chains[i];
-        if (!same_order(o)) continue;
+        if (o.join || !same_order(o)) continue;
         if (c.ownF) { c.offF = o.offF; c.ownF = 0; }
         if (c.ownS && o.sg == sg && o.sfrag == sfrag) { c.offS = o.offS; c.ownS = 0; }
         if (c.ownL && o.lg == lg) { c.offL = o.offL; c.ownL = 0; }
@@ -84,6 +85,26 @@ int plan_chain(Plan *p, const int order[3], int sg, int lg, int sfrag) {
     if (c.ownF) c.offF = take(size_t(c.oF) * c.R * c.R * c.KF);
     if (c.ownS) c.offS = take(size_t(sfrag ? round_up(c.oS * c.R, 32) : c.oS * c.R) * c.K2);
     if (c.ownL) c.offL = take(size_t(c.nL) * c.oL * c.R * c.R);
+    return p->nchains++;
+}
+
+int plan_join_chain(Plan *p) {
+    for (int i = 0; i < p->nchains; ++i)
+        if (p->chains[i].join) return i;
+    if (p->nchains == kMaxChains) return -1;
+    static const int kOrder[3] = {1, 2, 0};
+    Chain &c = p->chains[p->nchains];
+    describe_chain(p->in_modes, p->out_modes, p->rank, kOrder, &c);
+    c.sg = c.lg = c.R;
+    c.sfrag = 0;
+    c.join = 1;
+    c.ownF = c.ownS = c.ownL = 0;
+    const size_t e = size_t(p->elem), R2 = size_t(c.R) * c.R;
+    if (R2 * (1 + 16 * size_t(c.nL) + size_t(c.oF) * c.nF + size_t(c.oS) * c.nS) >> 31) return -1;
+    c.offF = p->packed_bytes;
+    c.offL = c.offF + kJoinHeader + e * R2;                 // J1: G1's fragments
+    c.offS = c.offL + e * R2 * 16 * c.nL;                    // J2, then J3
+    p->packed_bytes = align256(c.offS + e * R2 * (size_t(c.oF) * c.nF + size_t(c.oS) * c.nS));
     return p->nchains++;
 }
 

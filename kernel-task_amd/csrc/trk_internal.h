@@ -35,6 +35,7 @@ struct Chain {
     int KF, K2;      // padded stage-1 and stage-2 contraction lengths
     int sg, lg;      // K-order groups of the Sk and Lk sections
     int sfrag;       // 1: Sk in 32x32x16 fragment order (trk_pack.hip)
+    int join;        // 1: the joined-core section (trk_pack.hip) at offF instead of the three
     int sxF, sxS, sxL;  // element strides of iF, iS, iL in a row of x
     int syF, syS, syL;  // element strides of f, s, l in a row of y
     size_t offF, offS, offL;  // byte offsets of Fk, Sk, Lk in the packed buffer
@@ -93,6 +94,11 @@ void describe_chain(const int in_modes[3], const int out_modes[3], int rank, con
                     Chain *chain);
 // index of the plan's chain with this order and K-order groups, added if new (-1: full)
 int plan_chain(Plan *plan, const int order[3], int sg, int lg, int sfrag);
+// index of the plan's joined-core section, added if new (-1: full)
+int plan_join_chain(Plan *plan);
+// The joined-core section: kJoinHeader bytes whose first float is the factor of the results,
+// R^2 zeros, then J1, J2 and J3 (trk_pack.hip).
+constexpr int kJoinHeader = 256;
 
 // Entry points a variant module (a generated table built at prepare time) exports, and the
 // layout check its loader applies: the module's sizeof(Plan) must equal the library's.

@@ -173,6 +173,9 @@ struct KCfg {
                              // one MFMA per K step, hold the SIMDs' issue priority while they
                              // run it (s_setprio), so that they finish before the waves with
                              // whole row tiles instead of after them, waiting on LDS alone
+    int JN;                  // 1: a joined-core tile (trk_join_kernel.h): TT tokens x (FC x SC)
+                             // pairs of output digits x all LC digits of G1, IC input digits
+                             // of G1 in LDS at a time, KS3 waves splitting the features
 };
 
 // K orders of the packed second- and last-core sections a variant reads (its chain's layout):
@@ -1557,9 +1560,9 @@ struct Shape {
 };
 constexpr KCfg tile(Shape s, int TT, int FC, int SC, int LC, int IC, int KS3, int NACC,
                     int WIDE = 0, int MF2 = 16, int NW = 4, int PIPE = 0, int S1 = 0,
-                    int XL = 0, int YM = 0, int SL = 0, int TP = 0) {
+                    int XL = 0, int YM = 0, int SL = 0, int TP = 0, int JN = 0) {
     return KCfg{s.dt, s.F, s.S, s.L, s.i0, s.i1, s.i2, s.o0, s.o1, s.o2, s.R,
-                TT, FC, SC, LC, IC, KS3, NACC, WIDE, MF2, NW, PIPE, S1, XL, YM, SL, TP};
+                TT, FC, SC, LC, IC, KS3, NACC, WIDE, MF2, NW, PIPE, S1, XL, YM, SL, TP, JN};
 }
 
 #define TRK_ENTRY(CFG, TMIN, TMAX) \
@@ -1580,7 +1583,8 @@ inline int register_entries(Plan *plan, const Entry *entries, int count) {
             continue;
         if (plan->nvariants == kMaxVariants) break;
         const int order[3] = {k.F, k.S, k.L};
-        const int chain = plan_chain(plan, order, s_group(k), l_group(k), s_frag(k));
+        const int chain = k.JN ? plan_join_chain(plan)
+                               : plan_chain(plan, order, s_group(k), l_group(k), s_frag(k));
         if (chain < 0) continue;
         Variant &v = plan->variants[plan->nvariants++];
         v.kind = TRK_KERNEL_MFMA;
@@ -1597,7 +1601,11 @@ inline int register_entries(Plan *plan, const Entry *entries, int count) {
         v.launch = e.launch;
         v.launch_pair = e.launch_pair;
         v.xcd_local = k.XL;
-        if (k.WIDE) {
+        if (k.JN) {
+            std::snprintf(v.name, sizeof(v.name), "ring3_join%s<%d%d%d,%d,%d,%d,%d,%d,%d,%d>",
+                          k.NW == 8 ? "_w8" : "", k.F, k.S, k.L, k.TT, k.FC, k.SC, k.LC, k.IC,
+                          k.KS3, k.NACC);
+        } else if (k.WIDE) {
             char s1[8] = "";
             if (k.S1) std::snprintf(s1, sizeof(s1), "_s%d", k.S1);
             std::snprintf(v.name, sizeof(v.name),

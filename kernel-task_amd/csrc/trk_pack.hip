@@ -18,6 +18,7 @@
 #include <algorithm>
 
 #include "trk_internal.h"
+#include "trk_types.h"
 
 namespace trk {
 namespace {
@@ -33,19 +34,20 @@ struct PackArgs {
     size_t nFk, nSk, nLk;  // element counts of the three sections
 };
 
-template <typename W>
+// N: 32 bits where the chain's sections have fewer than 2^31 elements (the index arithmetic is a
+// chain of divisions, several times as long in 64 bits)
+template <typename W, typename N>
 __global__ void __launch_bounds__(256) pack_chain_kernel(const W *__restrict__ gF,
                                                          const W *__restrict__ gS,
                                                          const W *__restrict__ gL,
                                                          W *__restrict__ Fk, W *__restrict__ Sk,
                                                          W *__restrict__ Lk, PackArgs a) {
-    const size_t total = a.nFk + a.nSk + a.nLk;
+    const N nFk = N(a.nFk), nSk = N(a.nSk), total = N(a.nFk + a.nSk + a.nLk);
     const int R = a.R;
-    for (size_t d = blockIdx.x * size_t(blockDim.x) + threadIdx.x; d < total;
-         d += size_t(gridDim.x) * blockDim.x) {
-        if (d < a.nFk) {
+    for (N d = blockIdx.x * N(blockDim.x) + threadIdx.x; d < total; d += N(gridDim.x) * blockDim.x) {
+        if (d < nFk) {
             const int iF = int(d % a.KF);
-            size_t rest = d / a.KF;
+            N rest = d / a.KF;
             const int r2 = int(rest % R);
             rest /= R;
             const int r1 = int(rest % R);
@@ -55,12 +57,12 @@ __global__ void __launch_bounds__(256) pack_chain_kernel(const W *__restrict__ g
                 v = gF[a.forward ? core_index(r1, f, iF, r2, a.oF, a.nF, a.Rc)
                                  : core_index(r2, f, iF, r1, a.oF, a.nF, a.Rc)];
             Fk[d] = v;
-        } else if (d < a.nFk + a.nSk) {
-            const size_t e = d - a.nFk;
+        } else if (d < nFk + nSk) {
+            const N e = d - nFk;
             int k, row;
             if (a.sfrag) {  // [tile][k / 16][lane][8]
                 const int lane = int(e / 8 % 64), ks = a.K2 / 16;
-                const size_t rest = e / 512;
+                const N rest = e / 512;
                 k = int(rest % ks) * 16 + lane / 32 * 8 + int(e % 8);
                 row = int(rest / ks) * 32 + lane % 32;
             } else {
@@ -78,10 +80,10 @@ __global__ void __launch_bounds__(256) pack_chain_kernel(const W *__restrict__ g
             }
             Sk[e] = v;
         } else {
-            const size_t e = d - a.nFk - a.nSk;
-            const int kk = int(e % (size_t(R) * R)), span = a.lg * R, rem = kk % span;
+            const N e = d - nFk - nSk;
+            const int kk = int(e % N(R * R)), span = a.lg * R, rem = kk % span;
             const int r1 = rem / a.lg, r3 = kk / span * a.lg + rem % a.lg;
-            size_t rest = e / (size_t(R) * R);
+            N rest = e / N(R * R);
             const int l = int(rest % a.oL);
             const int iL = int(rest / a.oL);
             W v = W(0);
@@ -98,6 +100,7 @@ int pack_all(const Plan &plan, const void *const g[3], void *packed, hipStream_t
     char *base = static_cast<char *>(packed);
     for (int ci = 0; ci < plan.nchains; ++ci) {
         const Chain &c = plan.chains[ci];
+        if (c.join) continue;
         PackArgs a;
         a.R = c.R;
         a.Rc = plan.core_rank;
@@ -119,7 +122,8 @@ int pack_all(const Plan &plan, const void *const g[3], void *packed, hipStream_t
         const size_t total = a.nFk + a.nSk + a.nLk;
         if (total == 0) continue;
         const int blocks = int(std::min<size_t>((total + 255) / 256, 4096));
-        hipLaunchKernelGGL(pack_chain_kernel<W>, dim3(blocks), dim3(256), 0, stream,
+        hipLaunchKernelGGL((total >> 31 ? &pack_chain_kernel<W, size_t> : &pack_chain_kernel<W, unsigned>),
+                           dim3(blocks), dim3(256), 0, stream,
                            static_cast<const W *>(g[c.order[0]]),
                            static_cast<const W *>(g[c.order[1]]),
                            static_cast<const W *>(g[c.order[2]]),
@@ -132,11 +136,147 @@ int pack_all(const Plan &plan, const void *const g[3], void *packed, hipStream_t
     return TRK_OK;
 }
 
+// The joined-core section (trk_join_kernel.h): [header][R^2 zeros][J1][J2][J3].
+//   J1[i][step][lane][8] = G1[a,p,i,b] as the formation's B fragments: column p = lane % 16 (zero
+//                          at or past oP), K position 8 g + u of lane group g = lane / 16 being
+//                          (a, b) in the order two results of the join (rows 4 g + u % 4) make a
+//                          K step; fp32 stores u in two planes of four ([u / 4][lane][u % 4])
+//   J2[q][j][b][c] = G2[b,q,j,c]
+//   J3[r][k][a][c] = G3[c,r,k,a]
+// fp16 cores are scaled by a power of two that brings the largest magnitude of each into [1/2, 1),
+// which changes no bits but the exponent (values more than 2^13 below the largest become
+// subnormal), and the header's first float is the factor that undoes it on the fp32 sums:
+// products of two and three cores are formed in the cores' type, and cores far from 1 would leave
+// fp16's range there. The header's next 3 x kPeaks floats are the largest magnitudes of the
+// cores' parts (infinite where a part holds an infinity or a NaN). bf16 and fp32 have the range.
+struct JoinArgs {
+    int R, Rc, nI, nJ, nK, oP, oQ, oR;
+    unsigned nJ1, nJ2, nJ3;  // (plan_join_chain keeps the section below 2^31 elements)
+};
+
+constexpr int kPeaks = 16;  // workgroups per core that look for its largest magnitude
+static_assert((1 + 3 * kPeaks) * 4 <= kJoinHeader, "the peaks fit the header");
+
+template <int DT>
+__global__ void __launch_bounds__(1024) join_peak_kernel(
+    const typename Elem<DT>::T *__restrict__ g1, const typename Elem<DT>::T *__restrict__ g2,
+    const typename Elem<DT>::T *__restrict__ g3, size_t n1, size_t n2, size_t n3, float *peaks) {
+    const typename Elem<DT>::T *g = blockIdx.y == 0 ? g1 : blockIdx.y == 1 ? g2 : g3;
+    const size_t n = blockIdx.y == 0 ? n1 : blockIdx.y == 1 ? n2 : n3;
+    float m = 0.0f;
+#pragma unroll 8
+    for (size_t i = blockIdx.x * 1024 + threadIdx.x; i < n; i += 1024 * kPeaks) {
+        const float v = fabsf(Elem<DT>::to_f32(g[i]));
+        m = v <= m ? m : v <= 3.4028234e38f ? v : INFINITY;
+    }
+    __shared__ float part[1024];
+    part[threadIdx.x] = m;
+    __syncthreads();
+    for (int w = 512; w > 0; w /= 2) {
+        if (threadIdx.x < w) part[threadIdx.x] = fmaxf(part[threadIdx.x], part[threadIdx.x + w]);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) peaks[blockIdx.y * kPeaks + blockIdx.x] = part[0];
+}
+
+// The power of two just above the largest of a core's peaks (0 if that is 0 or not finite).
+__device__ inline int join_exponent(const float *peaks) {
+    float m = 0.0f;
+    for (int i = 0; i < kPeaks; ++i) m = fmaxf(m, peaks[i]);
+    int e = 0;
+    if (m > 0.0f && m <= 3.4028234e38f) frexpf(m, &e);
+    return e;
+}
+
+template <int DT>
+__global__ void __launch_bounds__(256) join_pack_kernel(
+    const typename Elem<DT>::T *__restrict__ g1, const typename Elem<DT>::T *__restrict__ g2,
+    const typename Elem<DT>::T *__restrict__ g3, char *__restrict__ out, JoinArgs a) {
+    using E = Elem<DT>;
+    using T = typename E::T;
+    int exponents[3] = {0, 0, 0};
+    if constexpr (DT == TRK_DTYPE_F16)
+        for (int k = 0; k < 3; ++k)
+            exponents[k] = join_exponent(reinterpret_cast<const float *>(out) + 1 + k * kPeaks);
+    const int R = a.R, R2 = R * R;
+    T *dst = reinterpret_cast<T *>(out + kJoinHeader);
+    const unsigned total = R2 + a.nJ1 + a.nJ2 + a.nJ3;
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        *reinterpret_cast<float *>(out) = ldexpf(1.0f, exponents[0] + exponents[1] + exponents[2]);
+    for (unsigned d = blockIdx.x * blockDim.x + threadIdx.x; d < total; d += gridDim.x * blockDim.x) {
+        float v = 0.0f;
+        int core = 0;
+        if (d < unsigned(R2)) {
+        } else if (d < R2 + a.nJ1) {
+            const unsigned e = d - R2;
+            const int in = int(e % 512), s = int(e / 512 % (R2 / 32)), i = int(e / 512 / (R2 / 32));
+            const int lane = sizeof(T) == 2 ? in / 8 : in % 256 / 4;
+            const int u = sizeof(T) == 2 ? in % 8 : in / 256 * 4 + in % 4;
+            const int p = lane % 16, g = lane / 16;
+            const int ca = R == 8 ? 4 * s + u / 4 * 2 + g / 2 : 2 * s + u / 4;
+            const int cb = R == 8 ? 4 * (g % 2) + u % 4 : 4 * g + u % 4;
+            if (p < a.oP && ca < a.Rc && cb < a.Rc)
+                v = E::to_f32(g1[core_index(ca, p, i, cb, a.oP, a.nI, a.Rc)]);
+        } else if (d < R2 + a.nJ1 + a.nJ2) {
+            const unsigned e = d - R2 - a.nJ1;
+            const int cc = int(e % R), cb = int(e / R % R), j = int(e / R2 % a.nJ);
+            const int q = int(e / R2 / a.nJ);
+            core = 1;
+            if (cb < a.Rc && cc < a.Rc)
+                v = E::to_f32(g2[core_index(cb, q, j, cc, a.oQ, a.nJ, a.Rc)]);
+        } else {
+            const unsigned e = d - R2 - a.nJ1 - a.nJ2;
+            const int cc = int(e % R), ca = int(e / R % R), k = int(e / R2 % a.nK);
+            const int r = int(e / R2 / a.nK);
+            core = 2;
+            if (ca < a.Rc && cc < a.Rc)
+                v = E::to_f32(g3[core_index(cc, r, k, ca, a.oR, a.nK, a.Rc)]);
+        }
+        dst[d] = E::from_f32(ldexpf(v, core == 0   ? -exponents[0]
+                                       : core == 1 ? -exponents[1]
+                                                   : -exponents[2]));
+    }
+}
+
+template <int DT>
+int pack_join(const Plan &plan, const Chain &c, const void *const g[3], void *packed,
+              hipStream_t stream) {
+    using T = typename Elem<DT>::T;
+    char *out = static_cast<char *>(packed) + c.offF;
+    const unsigned R2 = c.R * c.R;
+    const T *t[3] = {static_cast<const T *>(g[0]), static_cast<const T *>(g[1]),
+                     static_cast<const T *>(g[2])};
+    if constexpr (DT == TRK_DTYPE_F16) {
+        size_t n[3];
+        for (int k = 0; k < 3; ++k)
+            n[k] = size_t(plan.core_rank) * plan.core_rank * plan.in_modes[k] * plan.out_modes[k];
+        hipLaunchKernelGGL(join_peak_kernel<DT>, dim3(kPeaks, 3), dim3(1024), 0, stream, t[0], t[1],
+                           t[2], n[0], n[1], n[2], reinterpret_cast<float *>(out) + 1);
+    }
+    JoinArgs a{c.R, plan.core_rank,
+               plan.in_modes[0], plan.in_modes[1], plan.in_modes[2],
+               plan.out_modes[0], plan.out_modes[1], plan.out_modes[2],
+               R2 * 16 * plan.in_modes[0], R2 * plan.in_modes[1] * plan.out_modes[1],
+               R2 * plan.in_modes[2] * plan.out_modes[2]};
+    const unsigned total = R2 + a.nJ1 + a.nJ2 + a.nJ3;
+    hipLaunchKernelGGL(join_pack_kernel<DT>, dim3(std::min(total / 256 + 1, 4096u)), dim3(256), 0,
+                       stream, t[0], t[1], t[2], out, a);
+    return check_hip(hipGetLastError(), "trk_pack: launch");
+}
+
 }  // namespace
 
 int launch_pack(const Plan &plan, const void *g1, const void *g2, const void *g3, void *packed,
                 hipStream_t stream) {
     const void *g[3] = {g1, g2, g3};
+    for (int ci = 0; ci < plan.nchains; ++ci) {
+        const Chain &c = plan.chains[ci];
+        if (!c.join) continue;
+        const int st = plan.dtype == TRK_DTYPE_F16    ? pack_join<TRK_DTYPE_F16>(plan, c, g, packed, stream)
+                       : plan.dtype == TRK_DTYPE_BF16 ? pack_join<TRK_DTYPE_BF16>(plan, c, g, packed, stream)
+                                                      : pack_join<TRK_DTYPE_F32>(plan, c, g, packed, stream);
+        if (st != TRK_OK) return st;
+    }
     if (plan.elem == 4) return pack_all<uint32_t>(plan, g, packed, stream);
     return pack_all<uint16_t>(plan, g, packed, stream);
 }

@@ -161,7 +161,8 @@ class Plan:
 
     @property
     def has_mfma(self) -> bool:
-        return any(v["kind"] == "mfma" for v in self.variants())
+        # (the MFMA variants come last: one description settles it)
+        return any(self.describe(v)["kind"] == "mfma" for v in reversed(range(self.variant_count)))
 
     def load_module(self, path) -> int:
         """Add the variants of a variant module (trk_plan_load_module); returns how many.

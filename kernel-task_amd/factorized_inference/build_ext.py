@@ -40,9 +40,16 @@ HIPCC_FLAGS = [
 ]
 
 
-# Per-source additions to HIPCC_FLAGS (the two MFMA kernel families are separate
-# translation units so that each can be tuned on its own).
-FILE_FLAGS: dict[str, list[str]] = {}
+def file_flags(src: Path) -> list[str]:
+    """HIPCC_FLAGS of one source. The joined-core tiles (csrc/trk_join_kernel.h) hold up to 400
+    registers a lane: with accumulators allowed in the accumulation half of the register file
+    they need no copies between the halves, where the VGPR form of the MFMAs copies its operands
+    there and back (measured at 14336 -> 4096 R16, T=2048, 256 tokens a workgroup: 421 us against
+    866). The other kernels fit the VGPR half."""
+    if not src.name.startswith("trk_gen_join_"):
+        return HIPCC_FLAGS
+    k = HIPCC_FLAGS.index("-amdgpu-mfma-vgpr-form=1")
+    return HIPCC_FLAGS[:k - 1] + HIPCC_FLAGS[k + 1:]
 
 
 def sources() -> list[Path]:
@@ -79,7 +86,7 @@ def build(verbose: bool = False, jobs: int = 8, incremental: bool = False) -> Pa
         if (incremental and obj.exists() and report.exists()
                 and obj.stat().st_mtime > max(_newest_dependency(), src.stat().st_mtime)):
             return obj
-        cmd = [hipcc, *HIPCC_FLAGS, *FILE_FLAGS.get(src.name, []),
+        cmd = [hipcc, *file_flags(src),
                "-Rpass-analysis=kernel-resource-usage", "-c", str(src), "-o", str(obj)]
         if verbose:
             print(" ".join(cmd), flush=True)

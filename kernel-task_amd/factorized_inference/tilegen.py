@@ -108,12 +108,15 @@ class Tile:
     #                stage 1 (LDS-staged) (KCfg::SL)
     TP: int = 0    # 1: the tail waves of a pair-and-tail stage 2 hold the issue priority while
     #                they run it (KCfg::TP; tiles with tail waves only)
+    JN: int = 0    # 1: a joined-core tile (csrc/trk_join_kernel.h): TT tokens x (FC x SC) pairs
+    #                of second- and third-core output digits x all of the first core's, IC input
+    #                digits of the first core in LDS at a time, KS3 waves splitting the features
 
     def args(self) -> str:
         """Arguments of tile(shape, ...) in the variant tables."""
         a = [self.TT, self.FC, self.SC, self.LC, self.IC, self.KS3, self.NACC]
         # each optional argument is spelled out when it or any later one differs from its default
-        tail = [self.PIPE, self.S1, self.XL, self.YM, self.SL, self.TP]
+        tail = [self.PIPE, self.S1, self.XL, self.YM, self.SL, self.TP, self.JN]
         last = max((i for i, v in enumerate(tail) if v), default=-1)
         if last >= 0 or (self.WIDE, self.MF2, self.NW) != (0, 16, 4):
             a += [self.WIDE, self.MF2, self.NW]
@@ -259,9 +262,53 @@ def pitch32(k: int) -> int:
     return k + 8
 
 
+JOIN_ORDER = (1, 2, 0)  # the joined family contracts G2 with G3, then G1, then x
+
+
+def join_geometry(shape: ShapeDecl, order: tuple, t: Tile) -> dict:
+    """geometry() of a joined-core tile (struct JoinGeo in trk_join_kernel.h)."""
+    (ni, nj, nk), (p, q, r), R = shape.ins, shape.outs, shape.rank
+    eb, ks, mt = ELEM_BYTES[shape.dtype], R * R // 32, t.TT // 16
+    qw = t.NW // t.KS3 if t.KS3 and t.NW % t.KS3 == 0 else 1
+    pairs = t.FC * t.SC
+    nq, shared = cdiv(pairs, qw), t.KS3 == 1
+    slices = t.FC * nj * R * R + t.SC * nk * (R * R + 16)
+    x_chunk = mt * 512 + (0 if shared else 16 // eb)
+    lds = max(eb * (slices + R * R + 2 * ks * 512 + 2 * t.KS3 * x_chunk),
+              min(mt, 4) * 16 * (pairs * 16 + 4) * 4 if shared else t.NW * nq * mt * 1024)
+    # registers of the arrays: accumulators, the joined slice, x in flight, G1's fragments, a
+    # formed tile and addresses
+    xf = mt + 2 * cdiv(mt, t.NW if shared else 1)  # read from LDS, two steps in flight
+    vgprs = (nq * mt * 4 + (nq * 2 + 1) * ks * 2 * eb + xf * 2 * eb + nq * (8 + 2 * eb)
+             + cdiv(mt, t.NW if shared else 1) + 24)
+    g = {"LDS_BYTES": lds, "NBLK": cdiv(q, t.FC) * cdiv(r, t.SC), "TAIL": False,
+         "join_vgprs": vgprs, "NQ": nq}
+    per_simd = 512 // max(1, t.NACC * t.NW // 4)
+    checks = [
+        (tuple(order) == JOIN_ORDER, "the joined family joins G2 and G3"),
+        (R in (8, 16), "joined tiles are written for ring ranks 8 and 16"),
+        (p <= 16 and t.LC == p, "a joined tile holds all first-core outputs in 16 columns"),
+        (nj * nk % 8 == 0 and nj * nk >= 32 and ni * nj * nk % (16 // eb) == 0,
+         "x is read 8 features at a time"),
+        (ni % 2 == 0 and t.IC == 1, "steps of one first-core digit, in pairs"),
+        (max(nq, t.SC) % min(nq, t.SC) == 0, "a wave's pairs are whole rows or parts of one"),
+        (t.NW in (4, 8) and t.KS3 >= 1 and t.NW % t.KS3 == 0, "KS3 must divide the waves"),
+        (t.TT > 0 and t.TT % 16 == 0, "tokens come in tiles of 16"),
+        (cdiv(nj * nk, 32) % t.KS3 == 0, "the waves take equal shares of the chunks"),
+        (pairs % qw == 0 and t.FC <= q and t.SC <= r, "pairs must split over the waves"),
+        (t.NACC in (1, 2) and t.NACC * t.NW <= 8, "at most two waves per SIMD"),
+        (lds * t.NACC <= LDS_LIMIT, f"LDS {lds} B exceeds 160 KB per CU"),
+        (vgprs <= per_simd, "joined tile needs too many registers"),
+    ]
+    g["reject"] = next((why for ok, why in checks if not ok), "")
+    return g
+
+
 def geometry(shape: ShapeDecl, order: tuple, t: Tile) -> dict:
     """The kernel's compile-time geometry (struct Geo) for one tile, with the reason the
     kernel would reject it ("" when it compiles). Mirrors the static_asserts of Geo."""
+    if t.JN:
+        return join_geometry(shape, order, t)
     c, R = chain_of(shape, order), shape.rank
     R2 = R * R
     eb = ELEM_BYTES[shape.dtype]
@@ -598,6 +645,7 @@ def candidates(shape: ShapeDecl, order: tuple | None = None,
     return out
 
 
+_JOIN_NAME = re.compile(r"ring3_join(_w8)?<(\d)(\d)(\d),(\d+),(\d+),(\d+),(\d+),(\d+),(\d+),(\d+)>")
 _VARIANT_NAME = re.compile(r"ring3_mfma(?:_wide(\d)(x32)?(w8)?(p2?)?(?:_s(\d+))?|(_w8)?(_p2?)?)"
                            r"(_xl|_x[24])?(_g)?(_sl)?(_tp)?<(\d)(\d)(\d),"
                            r"(\d+),(\d+),(\d+),(\d+),(\d+),(\d+),(\d+)>")
@@ -605,6 +653,10 @@ _VARIANT_NAME = re.compile(r"ring3_mfma(?:_wide(\d)(x32)?(w8)?(p2?)?(?:_s(\d+))?
 
 def parse_variant_name(name: str) -> tuple[tuple, Tile]:
     """(chain order, tile) of an MFMA variant from its name in the plan (trk_variant_info)."""
+    j = _JOIN_NAME.fullmatch(name)
+    if j:
+        return (tuple(int(j.group(i)) for i in (2, 3, 4)),
+                Tile(*(int(j.group(i)) for i in range(5, 12)), NW=8 if j.group(1) else 4, JN=1))
     m = _VARIANT_NAME.fullmatch(name)
     if not m:
         raise ValueError(f"not an MFMA variant name: {name!r}")
@@ -684,6 +736,25 @@ def neighbours(shape: ShapeDecl, order: tuple, t: Tile) -> dict[str, Tile]:
     return out
 
 
+def join_candidates(shape: ShapeDecl) -> dict[str, Tile]:
+    """The joined-core tiles worth timing (extended search): waves that split the features of
+    1-4 output pairs at few tokens, and waves that share x over 4-16 pairs at many, two
+    workgroups a CU where they fit."""
+    small, large = (16, 32, 48, 64, 96, 128), (64, 96, 128, 192, 256)
+    kinds = [(tt, fc, sc, 4) for tt in small for fc, sc in ((1, 1), (2, 1), (1, 2), (3, 1), (1, 4))]
+    kinds += [(tt, fc, sc, 1) for tt in large for fc, sc in ((1, 4), (2, 4), (1, 8), (2, 8))]
+    out = {}
+    for tt, fc, sc, kw in kinds:
+        if shape.rank == 8 and tt < 48:  # the chains cost less there
+            continue
+        for wpc in (2, 1):
+            t = Tile(tt, fc, sc, shape.outs[0], 1, kw, wpc, JN=1)
+            if not join_geometry(shape, JOIN_ORDER, t)["reject"]:
+                out[f"join_t{tt}f{fc}s{sc}k{kw}w{wpc}"] = t
+                break
+    return out
+
+
 def search_candidates(shape: ShapeDecl, extended: bool = False) -> dict[str, tuple[tuple, Tile]]:
     """name -> (order, tile) over every searched order; tiles of an order other than the
     shape's own carry the suffix @FSL in their names."""
@@ -693,6 +764,9 @@ def search_candidates(shape: ShapeDecl, extended: bool = False) -> dict[str, tup
         tag = "" if order == first else "@" + order_tag(order)
         for name, t in candidates(shape, order, extended).items():
             out[name + tag] = (order, t)
+    if extended:
+        out |= {name + "@" + order_tag(JOIN_ORDER): (JOIN_ORDER, t)
+                for name, t in join_candidates(shape).items()}
     return out
 
 
@@ -713,14 +787,15 @@ def table(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = Fa
           extended: bool = False) -> list[tuple[str, tuple, Tile, int, int]]:
     """[(name, order, tile, t_min, t_max)] for one shape: the tuned winners when the shape
     has measurements, else every candidate with the rule's ranges (0, 0: index only).
-    A tuned entry's "extra" tiles are compiled index-only beside the winners (alternatives
-    a caller may route token counts to, such as the XCD-local tiles).
+    A tuned entry's "ranges" are its chain tiles, "joined" its joined-core tiles. Its "extra"
+    tiles are compiled index-only beside the winners (alternatives a caller may route token
+    counts to, such as the XCD-local tiles).
     all_candidates=True ignores the measurements (the autotuner's input)."""
     tuned = load_tuned() if tuned is None else tuned
     entry = None if all_candidates else tuned.get(shape.key)
     if entry:
         rows = [(r["name"], tuple(r.get("order", entry["order"])), Tile(**r["tile"]),
-                 r["t_min"], r["t_max"]) for r in entry["ranges"]]
+                 r["t_min"], r["t_max"]) for r in entry["ranges"] + entry.get("joined", [])]
         rows += [(r["name"], tuple(r.get("order", entry["order"])), Tile(**r["tile"]), 0, 0)
                  for r in entry.get("extra", [])]
         for name, order, t, _, _ in rows:
@@ -738,7 +813,7 @@ def table(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = Fa
         # stage 2 with the tail waves' issue priority (TP) and, for the register-resident
         # winners of 5 tokens or more, their neighbours (a local refinement)
         entry = tuned[shape.key]
-        for r in entry["ranges"] + entry.get("extra", []):
+        for r in entry["ranges"] + entry.get("joined", []) + entry.get("extra", []):
             order = tuple(r.get("order", entry["order"]))
             if order not in ORDERS:
                 continue
@@ -749,7 +824,7 @@ def table(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = Fa
             base, _, tag = name.partition("@")
             tag = "@" + tag if tag else ""
             found = [(name, tile)]
-            if extended:
+            if extended and not tile.JN:
                 found += [(base + suffix + tag, v)
                           for suffix, v in s1_variants(shape, order, tile).items()]
                 late = replace(tile, SL=1)
@@ -766,14 +841,16 @@ def table(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = Fa
     return [(n, o, t, *ranges.get(n, (0, 0))) for n, (o, t) in cands.items()]
 
 
-def _fn_name(shape: ShapeDecl) -> str:
-    return "mfma_register_gen_" + shape.key
+def _fn_name(shape: ShapeDecl, join: bool = False) -> str:
+    return ("join" if join else "mfma") + "_register_gen_" + shape.key
 
 
 def emit(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = False,
-         extended: bool = False) -> str:
+         extended: bool = False, join: bool = False) -> str:
+    """One translation unit: the shape's chain tiles, or (join) its joined-core tiles, which
+    build_ext compiles with other flags."""
     tuned = load_tuned() if tuned is None else tuned
-    rows = table(shape, tuned, all_candidates, extended)
+    rows = [r for r in table(shape, tuned, all_candidates, extended) if bool(r[2].JN) == join]
     orders = sorted({r[1] for r in rows}, key=lambda od: (od != choose_order(shape), od))
     i, o = shape.ins, shape.outs
     tuned_note = ("token ranges measured by kernel-task_amd/benchmarks/autotune.py"
@@ -785,7 +862,7 @@ def emit(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = Fal
         f"{shape.rank}, {shape.dtype}, chain order"
         f"{'s' if len(orders) > 1 else ''} "
         + ", ".join(f"({od[0]},{od[1]},{od[2]})" for od in orders) + f"; {tuned_note}.",
-        '#include "trk_mfma_kernel.h"',
+        f'#include "trk_{"join" if join else "mfma"}_kernel.h"',
         "",
         "namespace trk {",
         "namespace {",
@@ -797,14 +874,14 @@ def emit(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = Fal
                      f"{shape.rank}}};")
     lines += ["", "const Entry kEntries[] = {"]
     for name, od, t, lo, hi in rows:
-        macro = "TRK_ENTRY_PAIR" if shape.swiglu else "TRK_ENTRY"
+        macro = "TRK_ENTRY" + ("_JOIN" if t.JN else "") + ("_PAIR" if shape.swiglu else "")
         lines.append(f"    {macro}(tile(kShape{order_tag(od)}, {t.args()}), {lo}, {hi})  // {name}")
     lines += [
         "};",
         "",
         "}  // namespace",
         "",
-        f"int {_fn_name(shape)}(Plan *plan) {{",
+        f"int {_fn_name(shape, join)}(Plan *plan) {{",
         "    return register_entries(plan, kEntries, int(sizeof(kEntries) / sizeof(kEntries[0])));",
         "}",
         "",
@@ -834,7 +911,7 @@ def emit_module(shape: ShapeDecl) -> str:
                         "kernel-task_amd/factorized_inference/jit.py (tilegen.emit_module).")
 
 
-def emit_index(shapes: list[ShapeDecl]) -> str:
+def emit_index(shapes: list[ShapeDecl], joined: list[ShapeDecl] = []) -> str:
     lines = [
         "// Generated by kernel-task_amd/factorized_inference/tilegen.py; do not edit.",
         "// Registers the generated MFMA variant tables (one translation unit per shape).",
@@ -843,9 +920,10 @@ def emit_index(shapes: list[ShapeDecl]) -> str:
         "namespace trk {",
         "",
     ]
-    lines += [f"int {_fn_name(s)}(Plan *plan);" for s in shapes]
+    names = [_fn_name(s) for s in shapes] + [_fn_name(s, True) for s in joined]
+    lines += [f"int {n}(Plan *plan);" for n in names]
     lines += ["", "int mfma_register_generated(Plan *plan) {", "    int added = 0;"]
-    lines += [f"    added += {_fn_name(s)}(plan);" for s in shapes]
+    lines += [f"    added += {n}(plan);" for n in names]
     lines += ["    return added;", "}", "", "}  // namespace trk", ""]
     return "\n".join(lines)
 
@@ -857,15 +935,22 @@ def write_all(shapes: list[ShapeDecl] = DECLARED, out_dir: Path = GEN_DIR,
     rule ranges (for the autotuner) instead of the tuned winners."""
     out_dir.mkdir(parents=True, exist_ok=True)
     tuned = load_tuned()
-    written = []
+    written, joined = [], []
     for s in shapes:
         p = out_dir / f"trk_gen_{s.key}.hip"
         text = emit(s, tuned, all_candidates, extended)
         if not p.exists() or p.read_text() != text:
             p.write_text(text)
         written.append(p)
+        if any(r[2].JN for r in table(s, tuned, all_candidates, extended)):
+            joined.append(s)
+            p = out_dir / f"trk_gen_join_{s.key}.hip"
+            text = emit(s, tuned, all_candidates, extended, join=True)
+            if not p.exists() or p.read_text() != text:
+                p.write_text(text)
+            written.append(p)
     index = out_dir / "trk_gen_index.hip"
-    text = emit_index(shapes)
+    text = emit_index(shapes, joined)
     if not index.exists() or index.read_text() != text:
         index.write_text(text)
     written.append(index)

@@ -1,0 +1,151 @@
+"""GPU parity of the joined-core tiles (csrc/trk_join_kernel.h) where they can go wrong: the edges
+of the token tile, the last, half-empty chunk of features (1920 -> 2880: 240 features of a first-core
+digit in chunks of 32), features of two second-core digits in one 16-wide tile, output modes below
+the 16 columns, zero-padded ranks, epilogues at every alignment of y, cores far from 1, and a captured
+launch. Against the float64 oracle, on the first and last rows (token rows are independent)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from factorized_inference import TRSpec, _lib, make_cores, prepare_optimized
+from factorized_inference.tr_kernel import current_stream_handle, forward_swiglu
+from gpu_util import check_result, oracle_y
+from oracle import ring_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {
+    "base_r8": ((8, 12, 20), (12, 10, 24), 8, torch.float16),
+    "base_r16": ((8, 12, 20), (12, 10, 24), 16, torch.float16),
+    "base_r8_fp32": ((8, 12, 20), (12, 10, 24), 8, torch.float32),
+    "llama_down_r16": ((16, 28, 32), (16, 16, 16), 16, torch.bfloat16),
+    "kv_r12": ((20, 16, 16), (8, 8, 16), 12, torch.bfloat16),
+    "down_r16": ((34, 32, 16), (16, 16, 20), 16, torch.bfloat16),
+    "gate_up_r8": ((20, 16, 16), (16, 34, 32), 8, torch.bfloat16),
+}
+# Relative 2-norm error: two roundings of the intermediates to the cores' type (each at most
+# eps / 2, about 0.3 eps in the mean square) and one of y, so below eps; fp32 sums of up to 17408
+# terms in runs of 8 to 544 MFMAs stay within 16 eps.
+REL = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7, torch.float32: 16 * 2.0 ** -23}
+
+
+def joined(run):
+    seen = {}
+    for i, v in enumerate(run.variants()):
+        if "join" in v["name"]:
+            seen.setdefault(v["name"], (i, v))
+    return list(seen.values())
+
+
+@pytest.mark.parametrize("name", SHAPES)
+def test_token_tile_edges(name):
+    ins, outs, rank, dtype = SHAPES[name]
+    spec = TRSpec(ins, outs, rank)
+    cores = make_cores(spec, device="cuda", dtype=dtype, seed=3)
+    run = prepare_optimized(cores, spec)
+    tiles = joined(run)
+    assert tiles
+    counts = {info["tile"][0]: (1, 15, info["tile"][0] - 1, info["tile"][0], info["tile"][0] + 1,
+                                2 * info["tile"][0] + 17) for _, info in tiles}
+    x_all = torch.randn(max(map(max, counts.values())), spec.in_features, device="cuda", dtype=dtype,
+                        generator=torch.Generator(device="cuda").manual_seed(4))
+    rows = sorted({r for c in counts.values() for t in c for r in (0, t // 2, t - 1)})
+    expected = dict(zip(rows, oracle_y(x_all[rows], cores, spec)))
+    for index, info in tiles:
+        for t in counts[info["tile"][0]]:
+            print("case:", name, info["name"], t, flush=True)
+            x = x_all[:t].clone()
+            y = run.run_variant(x, index)
+            rows = sorted({0, t // 2, t - 1})
+            want = np.stack([expected[r] for r in rows])
+            check_result(y[rows], want, dtype)
+            rel = orc.errors(y[rows].double().cpu().numpy(), want)["relative_l2_error"]
+            assert rel <= REL[dtype], rel
+            assert torch.isfinite(y).all()
+            assert torch.equal(y, run.run_variant(x, index))  # repeated calls are identical
+
+
+@pytest.mark.parametrize("name", ["base_r16", "base_r8_fp32", "down_r16"])
+def test_epilogues_at_every_alignment(name):
+    ins, outs, rank, dtype = SHAPES[name]
+    spec = TRSpec(ins, outs, rank)
+    cores = make_cores(spec, device="cuda", dtype=dtype, seed=5)
+    run = prepare_optimized(cores, spec)
+    lib, stream = _lib.load(), current_stream_handle(run.device_index)
+    t, n = 130, spec.out_features
+    x = torch.randn(t, spec.in_features, device="cuda", generator=torch.Generator(
+        device="cuda").manual_seed(6), dtype=dtype)
+    aux = torch.randn(t, n, device="cuda", dtype=dtype, generator=torch.Generator(
+        device="cuda").manual_seed(7))
+    for index, info in joined(run):
+        print("case:", name, info["name"], flush=True)
+        y32 = run.run_variant(x, index, _lib.EPI_F32)
+        assert torch.equal(run.run_variant(x, index), y32.to(dtype))
+        added = (aux.float() + y32).to(dtype)
+        gated = run.run_variant(x, index, _lib.EPI_SILU_MUL, aux)
+        for off in (0, 1, 2, 3):  # elements past an aligned buffer: runs of stores and single ones
+            out = torch.empty(t * n + off, device="cuda", dtype=dtype)[off:].view(t, n)
+            res = torch.empty(t * n + off, device="cuda", dtype=dtype)[off:].view(t, n).copy_(aux)
+            for epi, a, want in ((_lib.EPI_STORE, None, y32.to(dtype)), (_lib.EPI_ADD, res, added),
+                                 (_lib.EPI_SILU_MUL, res, gated), (_lib.EPI_ADD, out, added)):
+                if a is out:  # aux may be y itself
+                    out.copy_(aux)
+                code = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}[dtype]
+                _lib.check(lib.trk_forward_epilogue(
+                    run.plan.handle, index, run.packed.data_ptr(), x.data_ptr(), out.data_ptr(), t,
+                    epi, a.data_ptr() if a is not None else None, code, stream))
+                assert torch.equal(out, want), (epi, off)
+            f32 = torch.empty(t * n + off, device="cuda")[off:].view(t, n)
+            _lib.check(lib.trk_forward_epilogue(
+                run.plan.handle, index, run.packed.data_ptr(), x.data_ptr(), f32.data_ptr(), t,
+                _lib.EPI_F32, None, 0, stream))
+            assert torch.equal(f32, y32)
+
+
+@pytest.mark.parametrize("scales", [(1e-3, 1e-3, 1e-3), (30.0, 1e-3, 30.0), (0.0, 1.0, 1.0)])
+def test_fp16_cores_far_from_one(scales):
+    # products of two or three such cores leave fp16's range; packing keeps their exponents apart
+    spec = TRSpec(rank=16)
+    cores = [c * s for c, s in zip(make_cores(spec, device="cuda", dtype=torch.float16, seed=8), scales)]
+    run = prepare_optimized(cores, spec)
+    x = torch.randn(70, spec.in_features, device="cuda", dtype=torch.float16,
+                    generator=torch.Generator(device="cuda").manual_seed(9))
+    expected = oracle_y(x[:4], cores, spec)
+    norm = np.linalg.norm(expected)
+    for index, info in joined(run):
+        y = run.run_variant(x, index, _lib.EPI_F32)[:4].double().cpu().numpy()
+        # (the cores' own subnormal values carry fewer bits, in the oracle alike)
+        assert np.linalg.norm(y - expected) <= 2.0 ** -10 * norm, info["name"]
+
+
+def test_swiglu_pair_of_joined_tiles():
+    ins, outs, rank, dtype = SHAPES["gate_up_r8"]
+    spec = TRSpec(ins, outs, rank)
+    gate, up = (prepare_optimized(make_cores(spec, device="cuda", dtype=dtype, seed=s), spec)
+                for s in (10, 11))
+    for t in sorted({v["t_min"] for _, v in joined(gate)} | {1100}):
+        print("case:", gate.selected(t)["name"], t, flush=True)
+        x = torch.randn(t, spec.in_features, device="cuda", dtype=dtype,
+                        generator=torch.Generator(device="cuda").manual_seed(t))
+        assert torch.equal(forward_swiglu(gate, up, x), up.forward_silu_mul(x, gate.accumulate(x)))
+
+
+def test_captured_joined_launch_replays():
+    spec = TRSpec(rank=16)
+    cores = make_cores(spec, device="cuda", dtype=torch.float16, seed=12)
+    run = prepare_optimized(cores, spec)
+    x = torch.randn(200, spec.in_features, device="cuda", dtype=torch.float16)
+    assert "join" in run.selected(200)["name"]
+    run(x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = run(x)
+    for replay in range(4):
+        x.copy_(torch.randn(200, spec.in_features, device="cuda", dtype=torch.float16))
+        graph.replay()
+        eager = run(x.clone())
+        torch.cuda.synchronize()
+        assert torch.equal(y, eager), replay
