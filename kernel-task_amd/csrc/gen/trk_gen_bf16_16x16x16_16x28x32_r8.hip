@@ -14,10 +14,9 @@ const Entry kEntries[] = {
     TRK_ENTRY_PAIR(tile(kShape012, 1, 1, 28, 32, 4, 1, 2, 8, 32, 8, 2, 4, 0, 0, 1), 5, 16)  // ring3_mfma_wide8x32w8p2_s4_sl<012,1,1,28,32,4,1,2>
     TRK_ENTRY_PAIR(tile(kShape012, 1, 2, 28, 32, 4, 1, 2, 8, 32, 8, 1, 4), 17, 32)  // ring3_mfma_wide8x32w8p_s4<012,1,2,28,32,4,1,2>
     TRK_ENTRY_PAIR(tile(kShape012, 1, 2, 28, 32, 4, 2, 1, 8, 32, 8, 0, 4), 33, 64)  // ring3_mfma_wide8x32w8_s4<012,1,2,28,32,4,2,1>
-    TRK_ENTRY_PAIR(tile(kShape012, 1, 8, 28, 32, 2, 2, 1, 8, 32, 8, 1), 65, 256)  // wide8x32w8_f8sc28k2n1_ic2_p
-    TRK_ENTRY_PAIR(tile(kShape012, 1, 8, 28, 32, 2, 2, 1, 8, 32, 8, 1), 321, 448)  // wide8x32w8_f8sc28k2n1_ic2_p
-    TRK_ENTRY_PAIR(tile(kShape012, 1, 8, 28, 32, 2, 2, 1, 8, 32, 8, 1), 641, 1024)  // wide8x32w8_f8sc28k2n1_ic2_p
-    TRK_ENTRY_PAIR(tile(kShape012, 1, 8, 28, 32, 2, 2, 1, 8, 32, 8, 1), 1281, 1536)  // wide8x32w8_f8sc28k2n1_ic2_p
+    TRK_ENTRY_PAIR(tile(kShape012, 1, 8, 28, 32, 2, 2, 1, 8, 32, 8, 1), 65, 128)  // wide8x32w8_f8sc28k2n1_ic2_p
+    TRK_ENTRY_PAIR(tile(kShape012, 1, 8, 28, 32, 2, 2, 1, 8, 32, 8, 1), 193, 256)  // wide8x32w8_f8sc28k2n1_ic2_p
+    TRK_ENTRY_PAIR(tile(kShape012, 1, 8, 28, 32, 2, 2, 1, 8, 32, 8, 1), 321, 384)  // wide8x32w8_f8sc28k2n1_ic2_p
 };
 
 }  // namespace

@@ -13,7 +13,6 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape210, 1, 1, 8, 16, 4, 8, 1, 8, 32, 8, 0, 0, 0, 0, 1), 3, 8)  // ring3_mfma_wide8x32w8_sl<210,1,1,8,16,4,8,1>
     TRK_ENTRY(tile(kShape210, 1, 1, 16, 16, 2, 2, 1, 8, 32, 8, 1, 2), 9, 16)  // ring3_mfma_wide8x32w8p_s2<210,1,1,16,16,2,2,1>
     TRK_ENTRY(tile(kShape210, 1, 2, 16, 16, 2, 2, 1, 8, 32, 8, 1, 4, 0, 0, 1), 17, 32)  // ring3_mfma_wide8x32w8p_s4_sl<210,1,2,16,16,2,2,1>
-    TRK_ENTRY(tile(kShape210, 2, 2, 16, 16, 1, 2, 1, 8, 32, 8, 1, 0, 0, 0, 1), 33, 48)  // ring3_mfma_wide8x32w8p_sl<210,2,2,16,16,1,2,1>
 };
 
 }  // namespace

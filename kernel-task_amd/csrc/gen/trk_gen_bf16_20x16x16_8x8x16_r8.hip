@@ -15,8 +15,7 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape012, 1, 1, 8, 16, 8, 2, 1, 4, 32, 8, 1), 9, 32)  // wide4x32w8_t1k2n1_ic8_p
     TRK_ENTRY(tile(kShape012, 1, 2, 8, 16, 8, 1, 2, 4, 32, 8, 2), 33, 64)  // wide4x32w8_f2k1n2_ic8_p2
     TRK_ENTRY(tile(kShape012, 1, 2, 8, 16, 4, 1, 2, 4, 32, 8, 1), 65, 128)  // wide4x32w8_f2k1n2_ic4_p
-    TRK_ENTRY(tile(kShape012, 1, 2, 8, 16, 4, 1, 2, 4, 32, 4), 129, 768)  // wide4x32_f2k1n2_ic4
-    TRK_ENTRY(tile(kShape012, 1, 2, 8, 16, 4, 1, 2, 4, 32, 4), 1025, 1280)  // wide4x32_f2k1n2_ic4
+    TRK_ENTRY(tile(kShape012, 1, 2, 8, 16, 4, 1, 2, 4, 32, 4), 129, 384)  // wide4x32_f2k1n2_ic4
 };
 
 }  // namespace

@@ -12,7 +12,6 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape210, 1, 1, 2, 12, 4, 4, 1), 2, 2)  // t1_s2
     TRK_ENTRY(tile(kShape210, 1, 1, 5, 12, 4, 2, 1, 8, 32, 8, 1), 3, 4)  // wide8x32w8_sc5k2n1_ic4_p
     TRK_ENTRY(tile(kShape210, 1, 1, 10, 12, 4, 2, 1, 8, 32, 8, 0, 2, 0, 0, 0, 1), 5, 8)  // ring3_mfma_wide8x32w8_s2_tp<210,1,1,10,12,4,2,1>
-    TRK_ENTRY(tile(kShape210, 1, 2, 10, 12, 4, 2, 1, 8, 32, 8, 0, 4), 9, 16)  // ring3_mfma_wide8x32w8_s4<210,1,2,10,12,4,2,1>
     TRK_ENTRY(tile(kShape210, 2, 3, 5, 12, 2, 2, 1, 8, 32, 8), 0, 0)  // cover_t2f3_half
     TRK_ENTRY(tile(kShape210, 3, 1, 10, 12, 2, 2, 1, 8, 32, 8), 0, 0)  // cover_t3
 };

@@ -36,6 +36,7 @@ int join_register_gen_bf16_20x16x16_8x8x16_r8(Plan *plan);
 int join_register_gen_bf16_20x16x16_8x8x16_r16(Plan *plan);
 int join_register_gen_bf16_24x16x16_16x16x20_r8(Plan *plan);
 int join_register_gen_bf16_24x16x16_16x16x20_r16(Plan *plan);
+int join_register_gen_bf16_20x16x16_16x32x32_r8(Plan *plan);
 int join_register_gen_bf16_20x16x16_16x32x32_r16(Plan *plan);
 
 int mfma_register_generated(Plan *plan) {
@@ -72,6 +73,7 @@ int mfma_register_generated(Plan *plan) {
     added += join_register_gen_bf16_20x16x16_8x8x16_r16(plan);
     added += join_register_gen_bf16_24x16x16_16x16x20_r8(plan);
     added += join_register_gen_bf16_24x16x16_16x16x20_r16(plan);
+    added += join_register_gen_bf16_20x16x16_16x32x32_r8(plan);
     added += join_register_gen_bf16_20x16x16_16x32x32_r16(plan);
     return added;
 }

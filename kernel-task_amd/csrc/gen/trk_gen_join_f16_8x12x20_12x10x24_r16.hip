@@ -8,15 +8,17 @@ namespace {
 constexpr Shape kShape120{TRK_DTYPE_F16, 1, 2, 0, 8, 12, 20, 12, 10, 24, 16};
 
 const Entry kEntries[] = {
-    TRK_ENTRY_JOIN(tile(kShape120, 32, 1, 1, 12, 1, 4, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 17, 32)  // ring3_join<120,32,1,1,12,1,4,2>
-    TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 1, 12, 1, 4, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 33, 64)  // ring3_join<120,64,1,1,12,1,4,2>
-    TRK_ENTRY_JOIN(tile(kShape120, 80, 1, 1, 12, 1, 4, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 65, 80)  // ring3_join<120,80,1,1,12,1,4,2>
-    TRK_ENTRY_JOIN(tile(kShape120, 64, 2, 1, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 81, 128)  // ring3_join<120,64,2,1,12,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 96, 2, 1, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 129, 192)  // ring3_join<120,96,2,1,12,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 193, 256)  // ring3_join<120,128,1,2,12,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 12, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 257, 512)  // ring3_join<120,128,1,4,12,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 12, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 513, 1024)  // ring3_join<120,128,1,8,12,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 256, 1, 8, 12, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1025, 1073741824)  // ring3_join<120,256,1,8,12,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 32, 1, 1, 12, 1, 8, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 9, 32)  // ring3_join_w8<120,32,1,1,12,1,8,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 1, 12, 1, 8, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 33, 64)  // ring3_join_w8<120,64,1,1,12,1,8,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 1, 12, 1, 8, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 65, 96)  // ring3_join_w8<120,96,1,1,12,1,8,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 2, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 97, 128)  // ring3_join_w8<120,64,1,2,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 1, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 129, 256)  // ring3_join_w8<120,128,2,1,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 12, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 257, 512)  // ring3_join_w8<120,128,1,4,12,1,2,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 12, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 513, 1024)  // ring3_join_w8<120,128,1,8,12,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 192, 1, 8, 12, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1025, 1536)  // ring3_join_w8<120,192,1,8,12,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 256, 1, 8, 12, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1537, 2048)  // ring3_join<120,256,1,8,12,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 192, 1, 8, 12, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2049, 3072)  // ring3_join_w8<120,192,1,8,12,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 256, 1, 8, 12, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 3073, 1073741824)  // ring3_join<120,256,1,8,12,1,1,1>
 };
 
 }  // namespace

@@ -11,14 +11,14 @@ const Entry kEntries[] = {
     TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 1, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 81, 96)  // ring3_join<120,96,1,1,12,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 97, 128)  // ring3_join<120,64,1,2,12,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 80, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 129, 160)  // ring3_join<120,80,1,2,12,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 161, 192)  // ring3_join<120,96,1,2,12,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 112, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 193, 224)  // ring3_join<120,112,1,2,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 2, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 161, 192)  // ring3_join_w8<120,96,1,2,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 112, 1, 2, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 193, 224)  // ring3_join_w8<120,112,1,2,12,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 225, 256)  // ring3_join<120,128,1,2,12,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 80, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 257, 320)  // ring3_join<120,80,1,2,12,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 321, 384)  // ring3_join<120,96,1,2,12,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 112, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 385, 448)  // ring3_join<120,112,1,2,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 2, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 321, 384)  // ring3_join_w8<120,96,1,2,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 112, 1, 2, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 385, 448)  // ring3_join_w8<120,112,1,2,12,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 449, 512)  // ring3_join<120,128,1,2,12,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 112, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 513, 640)  // ring3_join<120,112,1,2,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 112, 1, 2, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 513, 640)  // ring3_join_w8<120,112,1,2,12,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 641, 1073741824)  // ring3_join<120,128,1,2,12,1,4,1>
 };
 

@@ -276,11 +276,11 @@ def join_geometry(shape: ShapeDecl, order: tuple, t: Tile) -> dict:
     x_chunk = mt * 512 + (0 if shared else 16 // eb)
     lds = max(eb * (slices + R * R + 2 * ks * 512 + 2 * t.KS3 * x_chunk),
               min(mt, 4) * 16 * (pairs * 16 + 4) * 4 if shared else t.NW * nq * mt * 1024)
-    # registers of the arrays: accumulators, the joined slice, x in flight, G1's fragments, a
-    # formed tile and addresses
-    xf = mt + 2 * cdiv(mt, t.NW if shared else 1)  # read from LDS, two steps in flight
-    vgprs = (nq * mt * 4 + (nq * 2 + 1) * ks * 2 * eb + xf * 2 * eb + nq * (8 + 2 * eb)
-             + cdiv(mt, t.NW if shared else 1) + 24)
+    # registers of the arrays: accumulators, the joined slice and G1's fragments, x read from LDS,
+    # two steps of it in flight, a formed tile, and addresses
+    rows = max(1, t.NW * (64 * 16 // (t.KS3 * 32 * eb))) if t.KS3 else 1  # x rows loaded at once
+    vgprs = (nq * mt * 4 + (nq * 2 + 1) * ks * 2 * eb + mt * 2 * eb + 9 * cdiv(t.TT, rows)
+             + nq * (8 + 2 * eb) + 28)
     g = {"LDS_BYTES": lds, "NBLK": cdiv(q, t.FC) * cdiv(r, t.SC), "TAIL": False,
          "join_vgprs": vgprs, "NQ": nq}
     per_simd = 512 // max(1, t.NACC * t.NW // 4)
@@ -737,20 +737,27 @@ def neighbours(shape: ShapeDecl, order: tuple, t: Tile) -> dict[str, Tile]:
 
 
 def join_candidates(shape: ShapeDecl) -> dict[str, Tile]:
-    """The joined-core tiles worth timing (extended search): waves that split the features of
-    1-4 output pairs at few tokens, and waves that share x over 4-16 pairs at many, two
-    workgroups a CU where they fit."""
+    """The joined-core tiles worth timing (extended search). Few tokens: waves that split the
+    features of 1-4 output pairs. Many: waves that share x over 4-16 pairs. Four waves of the
+    largest tile a register file holds suit calls that fill the chip several times over; eight
+    (one workgroup a CU) suit the calls of one or two rounds, where two waves a SIMD hide what
+    one of them waits for."""
     small, large = (16, 32, 48, 64, 96, 128), (64, 96, 128, 192, 256)
-    kinds = [(tt, fc, sc, 4) for tt in small for fc, sc in ((1, 1), (2, 1), (1, 2), (3, 1), (1, 4))]
-    kinds += [(tt, fc, sc, 1) for tt in large for fc, sc in ((1, 4), (2, 4), (1, 8), (2, 8))]
+    mid = (16, 32, 48, 64, 80, 96, 112, 128, 160, 192)
+    kinds = [(4, tt, fc, sc, 4) for tt in small for fc, sc in ((1, 1), (2, 1), (1, 2), (3, 1), (1, 4))]
+    kinds += [(4, tt, fc, sc, 1) for tt in large for fc, sc in ((1, 4), (2, 4), (1, 8), (2, 8))]
+    kinds += [(8, tt, fc, sc, kw) for tt in mid for kw, pairs in (
+        (8, ((1, 1), (1, 2))), (4, ((1, 2), (2, 1), (1, 4))), (2, ((1, 4), (1, 8), (2, 4))),
+        (1, ((1, 8), (2, 4), (2, 8), (4, 4)))) for fc, sc in pairs]
     out = {}
-    for tt, fc, sc, kw in kinds:
+    for nw, tt, fc, sc, kw in kinds:
         if shape.rank == 8 and tt < 48:  # the chains cost less there
             continue
         for wpc in (2, 1):
-            t = Tile(tt, fc, sc, shape.outs[0], 1, kw, wpc, JN=1)
+            t = Tile(tt, fc, sc, shape.outs[0], 1, kw, wpc, NW=nw, JN=1)
             if not join_geometry(shape, JOIN_ORDER, t)["reject"]:
-                out[f"join_t{tt}f{fc}s{sc}k{kw}w{wpc}"] = t
+                w8 = "w8" if nw == 8 else ""
+                out[f"join{w8}_t{tt}f{fc}s{sc}k{kw}w{wpc}"] = t
                 break
     return out
 
