@@ -11,8 +11,7 @@ const Entry kEntries[] = {
     TRK_ENTRY_PAIR(tile(kShape012, 1, 1, 5, 32, 8, 2, 2), 1, 2)  // mid_1of8_k2
     TRK_ENTRY_PAIR(tile(kShape012, 1, 1, 17, 32, 8, 2, 1, 8, 32, 8), 3, 8)  // wide8x32w8_t1k2n1_ic8
     TRK_ENTRY_PAIR(tile(kShape012, 1, 2, 17, 32, 8, 1, 2, 8, 32, 8), 9, 16)  // wide8x32w8_f2k1n2_ic8
-    TRK_ENTRY_PAIR(tile(kShape012, 1, 2, 17, 32, 4, 1, 2, 4, 32, 4), 17, 96)  // wide4x32_f2k1n2_ic4
-    TRK_ENTRY_PAIR(tile(kShape012, 1, 2, 17, 32, 4, 1, 2, 4, 32, 4), 129, 160)  // wide4x32_f2k1n2_ic4
+    TRK_ENTRY_PAIR(tile(kShape012, 1, 2, 17, 32, 4, 1, 2, 4, 32, 4), 17, 160)  // wide4x32_f2k1n2_ic4
 };
 
 }  // namespace

@@ -1,12 +1,11 @@
 // Generated by kernel-task_amd/factorized_inference/tilegen.py; do not edit.
-// r8_fp32: (8,12,20) -> (12,10,24), rank 8, f32, chain orders (2,1,0), (1,0,2); token ranges measured by kernel-task_amd/benchmarks/autotune.py.
+// r8_fp32: (8,12,20) -> (12,10,24), rank 8, f32, chain order (2,1,0); token ranges measured by kernel-task_amd/benchmarks/autotune.py.
 #include "trk_mfma_kernel.h"
 
 namespace trk {
 namespace {
 
 constexpr Shape kShape210{TRK_DTYPE_F32, 2, 1, 0, 8, 12, 20, 12, 10, 24, 8};
-constexpr Shape kShape102{TRK_DTYPE_F32, 1, 0, 2, 8, 12, 20, 12, 10, 24, 8};
 
 const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape210, 1, 1, 2, 6, 8, 8, 1, 0, 16, 8), 1, 1)  // t1_l6_s2_w8_k8
@@ -14,8 +13,6 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape210, 1, 1, 10, 12, 4, 4, 1, 8, 32, 8, 1), 3, 8)  // ring3_mfma_wide8x32w8p<210,1,1,10,12,4,4,1>
     TRK_ENTRY(tile(kShape210, 1, 2, 10, 12, 4, 4, 1, 8, 32, 8, 1), 9, 16)  // ring3_mfma_wide8x32w8p<210,1,2,10,12,4,4,1>
     TRK_ENTRY(tile(kShape210, 1, 3, 10, 12, 4, 4, 1, 8, 32, 8), 17, 32)  // wide8x32w8_f3k4n1_ic4
-    TRK_ENTRY(tile(kShape210, 1, 6, 10, 12, 2, 2, 1, 8, 32, 8, 1), 33, 64)  // wide8x32w8_f6k2n1_ic2_p
-    TRK_ENTRY(tile(kShape102, 1, 2, 12, 24, 2, 1, 2, 4, 32, 4), 65, 80)  // ring3_mfma_wide4x32<102,1,2,12,24,2,1,2>
     TRK_ENTRY(tile(kShape210, 2, 3, 10, 12, 1, 2, 1, 8, 32, 8, 1), 0, 0)  // cover_t2f3_p
 };
 

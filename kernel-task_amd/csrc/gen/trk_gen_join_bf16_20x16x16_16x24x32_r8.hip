@@ -15,7 +15,7 @@ const Entry kEntries[] = {
     TRK_ENTRY_JOIN(tile(kShape120, 160, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1281, 1536)  // ring3_join_w8<120,160,2,8,16,1,1,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1537, 2048)  // ring3_join_w8<120,128,2,8,16,1,1,1>
     TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2049, 3072)  // ring3_join_w8<120,192,2,8,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 160, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 3073, 1073741824)  // ring3_join_w8<120,160,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 3073, 1073741824)  // ring3_join_w8<120,128,2,8,16,1,1,1>
 };
 
 }  // namespace

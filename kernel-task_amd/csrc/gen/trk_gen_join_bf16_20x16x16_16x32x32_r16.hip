@@ -9,14 +9,23 @@ constexpr Shape kShape120{TRK_DTYPE_BF16, 1, 2, 0, 20, 16, 16, 16, 32, 32, 16};
 
 const Entry kEntries[] = {
     TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 33, 64)  // ring3_join_w8<120,64,1,4,16,1,2,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 65, 128)  // ring3_join_w8<120,128,1,4,16,1,2,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 65, 96)  // ring3_join_w8<120,96,1,4,16,1,2,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 97, 128)  // ring3_join_w8<120,128,1,4,16,1,2,1>
     TRK_ENTRY_JOIN(tile(kShape120, 192, 1, 4, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 129, 192)  // ring3_join<120,192,1,4,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 193, 256)  // ring3_join<120,128,1,8,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 192, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 257, 384)  // ring3_join<120,192,1,8,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 385, 512)  // ring3_join<120,256,1,8,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 160, 1, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 513, 640)  // ring3_join_w8<120,160,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 193, 256)  // ring3_join_w8<120,128,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 176, 1, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 257, 320)  // ring3_join_w8<120,176,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 192, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 321, 384)  // ring3_join<120,192,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 224, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 385, 448)  // ring3_join<120,224,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 449, 512)  // ring3_join<120,256,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 176, 1, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 513, 640)  // ring3_join_w8<120,176,1,8,16,1,1,1>
     TRK_ENTRY_JOIN(tile(kShape120, 192, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 641, 768)  // ring3_join<120,192,1,8,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 769, 1073741824)  // ring3_join<120,256,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 224, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 769, 896)  // ring3_join<120,224,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 897, 1024)  // ring3_join<120,256,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 192, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1025, 1152)  // ring3_join<120,192,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 224, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1153, 1280)  // ring3_join<120,224,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1281, 1536)  // ring3_join<120,256,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 224, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1537, 1792)  // ring3_join<120,224,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1793, 1073741824)  // ring3_join<120,256,1,8,16,1,1,1>
 };
 
 }  // namespace

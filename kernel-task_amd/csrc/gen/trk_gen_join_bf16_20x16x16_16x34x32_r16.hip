@@ -10,17 +10,25 @@ constexpr Shape kShape120{TRK_DTYPE_BF16, 1, 2, 0, 20, 16, 16, 16, 34, 32, 16};
 const Entry kEntries[] = {
     TRK_ENTRY_JOIN_PAIR(tile(kShape120, 48, 3, 1, 16, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 33, 48)  // ring3_join<120,48,3,1,16,1,4,1>
     TRK_ENTRY_JOIN_PAIR(tile(kShape120, 64, 3, 1, 16, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 49, 64)  // ring3_join<120,64,3,1,16,1,4,1>
-    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 80, 1, 1, 16, 1, 4, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 65, 80)  // ring3_join<120,80,1,1,16,1,4,2>
-    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 128, 1, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 81, 128)  // ring3_join_w8<120,128,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 96, 1, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 65, 96)  // ring3_join_w8<120,96,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 128, 1, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 97, 128)  // ring3_join_w8<120,128,1,8,16,1,1,1>
     TRK_ENTRY_JOIN_PAIR(tile(kShape120, 160, 1, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 129, 160)  // ring3_join_w8<120,160,1,8,16,1,1,1>
-    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 192, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 161, 192)  // ring3_join<120,192,1,8,16,1,1,1>
-    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 193, 256)  // ring3_join<120,256,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 192, 1, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 161, 192)  // ring3_join_w8<120,192,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 224, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 193, 224)  // ring3_join<120,224,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 225, 256)  // ring3_join<120,256,1,8,16,1,1,1>
     TRK_ENTRY_JOIN_PAIR(tile(kShape120, 128, 1, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 257, 384)  // ring3_join_w8<120,128,1,8,16,1,1,1>
     TRK_ENTRY_JOIN_PAIR(tile(kShape120, 160, 1, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 385, 448)  // ring3_join_w8<120,160,1,8,16,1,1,1>
-    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 192, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 449, 512)  // ring3_join<120,192,1,8,16,1,1,1>
-    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 513, 768)  // ring3_join<120,256,1,8,16,1,1,1>
-    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 192, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 769, 896)  // ring3_join<120,192,1,8,16,1,1,1>
-    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 897, 1073741824)  // ring3_join<120,256,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 192, 1, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 449, 512)  // ring3_join_w8<120,192,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 224, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 513, 640)  // ring3_join<120,224,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 641, 768)  // ring3_join<120,256,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 192, 1, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 769, 896)  // ring3_join_w8<120,192,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 224, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 897, 1024)  // ring3_join<120,224,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 240, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1025, 1152)  // ring3_join<120,240,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1153, 1280)  // ring3_join<120,256,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 224, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1281, 1536)  // ring3_join<120,224,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1537, 1792)  // ring3_join<120,256,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 240, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1793, 3072)  // ring3_join<120,240,1,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 256, 1, 8, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 3073, 1073741824)  // ring3_join<120,256,1,8,16,1,1,1>
 };
 
 }  // namespace

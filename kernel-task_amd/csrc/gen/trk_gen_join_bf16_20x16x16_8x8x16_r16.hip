@@ -13,11 +13,13 @@ const Entry kEntries[] = {
     TRK_ENTRY_JOIN(tile(kShape120, 80, 1, 1, 8, 1, 8, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 129, 160)  // ring3_join_w8<120,80,1,1,8,1,8,1>
     TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 1, 8, 1, 8, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 161, 192)  // ring3_join_w8<120,96,1,1,8,1,8,1>
     TRK_ENTRY_JOIN(tile(kShape120, 64, 2, 1, 8, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 193, 256)  // ring3_join<120,64,2,1,8,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 2, 8, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 257, 512)  // ring3_join_w8<120,128,1,2,8,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 2, 8, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 257, 384)  // ring3_join_w8<120,96,1,2,8,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 2, 8, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 385, 512)  // ring3_join_w8<120,128,1,2,8,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 8, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 513, 1024)  // ring3_join_w8<120,128,1,4,8,1,2,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 256, 1, 4, 8, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1025, 2048)  // ring3_join<120,256,1,4,8,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 2, 8, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1025, 1152)  // ring3_join_w8<120,96,1,2,8,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 8, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1153, 2048)  // ring3_join_w8<120,128,1,8,8,1,1,1>
     TRK_ENTRY_JOIN(tile(kShape120, 192, 1, 8, 8, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2049, 3072)  // ring3_join_w8<120,192,1,8,8,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 256, 1, 4, 8, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 3073, 1073741824)  // ring3_join<120,256,1,4,8,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 8, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 3073, 1073741824)  // ring3_join_w8<120,128,1,8,8,1,1,1>
 };
 
 }  // namespace

@@ -13,8 +13,9 @@ const Entry kEntries[] = {
     TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 4, 8, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 641, 768)  // ring3_join_w8<120,96,1,4,8,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 8, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 769, 1024)  // ring3_join_w8<120,128,1,4,8,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 8, 8, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1025, 1536)  // ring3_join_w8<120,96,1,8,8,1,2,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 8, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1537, 2048)  // ring3_join_w8<120,128,1,8,8,1,2,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 8, 8, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2049, 1073741824)  // ring3_join_w8<120,128,2,8,8,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 4, 8, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1537, 2048)  // ring3_join_w8<120,128,2,4,8,1,2,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 2, 8, 8, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2049, 3072)  // ring3_join_w8<120,96,2,8,8,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 8, 8, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 3073, 1073741824)  // ring3_join_w8<120,128,2,8,8,1,1,1>
 };
 
 }  // namespace

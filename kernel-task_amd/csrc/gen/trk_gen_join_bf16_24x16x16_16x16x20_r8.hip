@@ -9,14 +9,15 @@ constexpr Shape kShape120{TRK_DTYPE_BF16, 1, 2, 0, 24, 16, 16, 16, 16, 20, 8};
 
 const Entry kEntries[] = {
     TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 4, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 161, 192)  // ring3_join_w8<120,64,1,4,16,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 80, 1, 4, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 193, 224)  // ring3_join_w8<120,80,1,4,16,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 225, 384)  // ring3_join_w8<120,128,1,4,16,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 96, 2, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 385, 448)  // ring3_join_w8<120,96,2,4,16,1,2,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 449, 768)  // ring3_join_w8<120,128,2,4,16,1,2,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 4, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 769, 1536)  // ring3_join_w8<120,128,4,4,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 192, 4, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1537, 2048)  // ring3_join_w8<120,192,4,4,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 257, 384)  // ring3_join_w8<120,128,1,4,16,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 2, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 385, 512)  // ring3_join_w8<120,96,2,4,16,1,2,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 513, 768)  // ring3_join_w8<120,128,2,4,16,1,2,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 4, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 769, 1024)  // ring3_join_w8<120,96,4,4,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 112, 4, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1025, 1280)  // ring3_join_w8<120,112,4,4,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 4, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1281, 1536)  // ring3_join_w8<120,128,4,4,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 176, 4, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1537, 2048)  // ring3_join_w8<120,176,4,4,16,1,1,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 4, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2049, 3072)  // ring3_join_w8<120,128,4,4,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 192, 4, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 3073, 1073741824)  // ring3_join_w8<120,192,4,4,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 176, 4, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 3073, 1073741824)  // ring3_join_w8<120,176,4,4,16,1,1,1>
 };
 
 }  // namespace

@@ -10,16 +10,17 @@ constexpr Shape kShape120{TRK_DTYPE_BF16, 1, 2, 0, 34, 32, 16, 16, 16, 20, 16};
 const Entry kEntries[] = {
     TRK_ENTRY_JOIN(tile(kShape120, 32, 2, 1, 16, 1, 4, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 9, 32)  // ring3_join<120,32,2,1,16,1,4,2>
     TRK_ENTRY_JOIN(tile(kShape120, 64, 2, 1, 16, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 33, 64)  // ring3_join<120,64,2,1,16,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 96, 2, 1, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 65, 96)  // ring3_join_w8<120,96,2,1,16,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 2, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 97, 128)  // ring3_join_w8<120,128,1,2,16,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 129, 160)  // ring3_join_w8<120,128,1,4,16,1,2,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 64, 2, 1, 16, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 161, 192)  // ring3_join<120,64,2,1,16,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 2, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 65, 96)  // ring3_join_w8<120,96,1,2,16,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 112, 1, 2, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 97, 112)  // ring3_join_w8<120,112,1,2,16,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 1, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 113, 128)  // ring3_join_w8<120,128,2,1,16,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 64, 2, 1, 16, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 129, 192)  // ring3_join<120,64,2,1,16,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 193, 384)  // ring3_join_w8<120,128,1,4,16,1,2,1>
     TRK_ENTRY_JOIN(tile(kShape120, 192, 1, 4, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 385, 512)  // ring3_join<120,192,1,4,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 513, 640)  // ring3_join_w8<120,128,2,4,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 4, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 641, 1024)  // ring3_join<120,192,2,4,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 256, 2, 4, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1025, 1536)  // ring3_join<120,256,2,4,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 4, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1537, 2048)  // ring3_join<120,192,2,4,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 513, 896)  // ring3_join_w8<120,192,2,4,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 4, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 897, 1152)  // ring3_join<120,192,2,4,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 256, 2, 4, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1153, 1536)  // ring3_join<120,256,2,4,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1537, 1792)  // ring3_join_w8<120,192,2,4,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 4, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 1793, 2048)  // ring3_join<120,192,2,4,16,1,1,1>
     TRK_ENTRY_JOIN(tile(kShape120, 256, 2, 4, 16, 1, 1, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 2049, 1073741824)  // ring3_join<120,256,2,4,16,1,1,1>
 };
 

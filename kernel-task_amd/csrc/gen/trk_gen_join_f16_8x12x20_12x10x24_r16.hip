@@ -12,7 +12,8 @@ const Entry kEntries[] = {
     TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 1, 12, 1, 8, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 33, 64)  // ring3_join_w8<120,64,1,1,12,1,8,1>
     TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 1, 12, 1, 8, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 65, 96)  // ring3_join_w8<120,96,1,1,12,1,8,1>
     TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 2, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 97, 128)  // ring3_join_w8<120,64,1,2,12,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 1, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 129, 256)  // ring3_join_w8<120,128,2,1,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 2, 1, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 129, 192)  // ring3_join_w8<120,96,2,1,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 2, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 193, 256)  // ring3_join_w8<120,128,1,2,12,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 12, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 257, 512)  // ring3_join_w8<120,128,1,4,12,1,2,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 12, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 513, 1024)  // ring3_join_w8<120,128,1,8,12,1,1,1>
     TRK_ENTRY_JOIN(tile(kShape120, 192, 1, 8, 12, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1025, 1536)  // ring3_join_w8<120,192,1,8,12,1,1,1>

@@ -8,8 +8,10 @@ namespace {
 constexpr Shape kShape120{TRK_DTYPE_F32, 1, 2, 0, 8, 12, 20, 12, 10, 24, 8};
 
 const Entry kEntries[] = {
-    TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 1, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 81, 96)  // ring3_join<120,96,1,1,12,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 97, 128)  // ring3_join<120,64,1,2,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 1, 12, 1, 8, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 33, 64)  // ring3_join_w8<120,64,1,1,12,1,8,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 1, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 65, 96)  // ring3_join<120,96,1,1,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 112, 1, 1, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 97, 112)  // ring3_join<120,112,1,1,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 113, 128)  // ring3_join<120,64,1,2,12,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 80, 1, 2, 12, 1, 4, 1, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 129, 160)  // ring3_join<120,80,1,2,12,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 96, 1, 2, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 161, 192)  // ring3_join_w8<120,96,1,2,12,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 112, 1, 2, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 193, 224)  // ring3_join_w8<120,112,1,2,12,1,4,1>

@@ -24,18 +24,22 @@
 //   Wt   results ft = 0, 1 (16 features (j,k) each) make a K step of 32: lane group g holds
 //        features 4 g .. 4 g + 3 of both, and x is laid out in LDS in that order
 //
-// Work split: a workgroup owns TT tokens x (FC x SC) output pairs x all p. KW of its 4 waves
+// Work split: a workgroup owns TT tokens x (FC x SC) output pairs x all p. KW of its 4 or 8 waves
 // split the feature chunks (their partial sums meet in LDS at the end), the others the pairs:
-// KW = 4 with one or two pairs where token tiles are few and the chip has to be filled with
+// KW = 4 or 8 with one or two pairs where token tiles are few and the chip has to be filled with
 // narrow tiles, KW = 1 with up to 16 where it is full, as the waves then share x and G1's fragments.
-// The steps (chunk of 32 features, digit i) run in lockstep over two LDS buffers.
+// The steps (chunk of 32 features, digit i) run in lockstep over two LDS buffers. Four waves leave
+// a SIMD one wave of up to 512 registers, whose tile amortises formation best (large calls); eight
+// leave it two of half the size, and one issues while the other waits: 5120 -> 12288 R16 T=128 63 ->
+// 59 us, 1920 -> 2880 R16 T=32 9.6 -> 8.0 us, R8 T=1023 31.5 -> 28.8 us.
 //
-// What bounds it: matrix cores (2-3 times the dense product's work at rank 16: R^2 / TT of
-// formation), with one wave a SIMD, so every wait shows. Of 107 us at 14336 -> 4096, rank 16, 256
-// tokens, the MFMAs take 47; x through LDS (whose writes run at a third of the reads' rate) and
-// the join of each chunk most of the rest. Measured against the chains on the same card: 217 ->
-// 103 us there; 5120 -> 12288 R16 T=128 156 -> 63 us; 17408 -> 5120 R16 T=2048 12650 -> 739 us (1.2
-// PFLOP/s with the formation); 1920 -> 2880 R8 T=1023 51.7 -> 31.5 us, fp32 T=100 41.6 -> 39.8 us.
+// What bounds it: at KW = 1 matrix cores (2-3 times the dense product's work at rank 16: R^2 / TT
+// of formation) and the waits between them; at KW = 4 and 8, where every wave reads its own x and
+// all of G1's fragments, LDS as well. At 14336 -> 4096, rank 16, 256 tokens (94 us) a step's MFMAs
+// take about 770 clocks of a CU and its LDS traffic about 1200: 128 KB of reads at the 206 B/clk
+// measured, 40 KB of writes at 68. Measured against the chains on the same card: 217 -> 94 us
+// there; 5120 -> 12288 R16 T=128 153 -> 59 us; 17408 -> 5120 R16 T=2048 12700 -> 735 us (1.2 PFLOP/s
+// with the formation); 1920 -> 2880 R8 T=1023 51.7 -> 28.8 us, fp32 T=100 41.7 -> 37.5 us.
 #include "trk_mfma_kernel.h"
 
 namespace trk {
@@ -57,7 +61,8 @@ struct JoinGeo {
     static constexpr bool XS = KW == 1;           // the waves share x
     static constexpr int KS = R2 / 32;            // K steps of the formation
     static constexpr int NCH = cdiv(NJK, 32);     // chunks of 32 features
-    static constexpr int NR = NCH / KW;           // chunks a wave works through
+    static constexpr int NR = cdiv(NCH, KW);      // chunks a wave works through
+    static constexpr bool PAD = NR * KW * 32 != NJK;  // some are empty, or end early: zeros
     static constexpr int NST = NR * nI;           // steps: (chunk, digit of i)
     static constexpr int FRAG = 512;              // elements of one operand fragment
     static constexpr int GPT = cdiv(KS * FRAG / VPE, NT);  // G1 vectors per thread and step
@@ -89,7 +94,11 @@ struct JoinGeo {
     // replace them all
     static constexpr int P3K = R2 + 16;
     static constexpr int szJ2 = FC * nJ * R2, szJ3 = SC * nK * P3K, szG1 = KS * FRAG;
-    static constexpr int szX = MT * FRAG + (KW > 1 ? VPE : 0);  // one step's x of one chunk
+    // one step's x of one chunk: the rows loaded at once are stored without a branch (it would cut
+    // the step's schedule in two: 5120 -> 17408 R16 T=160, TT = 160 over 8 waves, 112 -> 106 us), so
+    // there is room for those past the tile
+    static constexpr int XROWS = XN * NW * RPI > TT ? XN * NW * RPI : TT;
+    static constexpr int szX = XROWS / 16 * FRAG + (KW > 1 ? VPE : 0);
     static constexpr int lJ3 = szJ2, lZ = lJ3 + szJ3, lG1 = lZ + R2, lX = lG1 + 2 * szG1;
     static constexpr int TILES = NQ * MT, TPW = cdiv(TILES, KW);  // y tiles, per storing wave
     // y through LDS (XS): [token][pair][p], a token's floats 4 words past a multiple of 64
@@ -105,7 +114,6 @@ struct JoinGeo {
     static_assert(NJK % 8 == 0 && NJK >= 32 && IN % VPE == 0, "x is read 8 features at a time");
     static_assert(nI % 2 == 0 && C.IC == 1, "steps of one digit of i, in pairs");
     static_assert(NQ % NRW == 0 && SC % NRW == 0, "a wave's pairs are whole rows or parts of one");
-    static_assert(NCH % KW == 0, "the waves take equal shares of the chunks");
     static_assert(TT % 16 == 0 && FC * SC % QW == 0 && NW % KW == 0 && FC <= oQ && SC <= oR,
                   "joined tile");
     static_assert(LDS_BYTES <= 160 * 1024, "joined tile exceeds the 160 KB of LDS");
@@ -269,15 +277,16 @@ __device__ __forceinline__ void join_unit(const typename Ops<C.dt>::E *__restric
     // the features of two lane groups of one result; in 32 bits, of one. The lane groups of row w
     // sit at slots g ^ x_swap(w), so that the 32 lanes one LDS pass serves read 32 different
     // 16-byte units.
-    // Byte offsets from the tile's first row (rows past the last token read the last one; their
-    // results are not stored).
+    // Byte offsets from the tile's first row (rows past the tile or the last token read the last one;
+    // their results are not stored).
     auto x_swap = [](int row) { return row / 8 % 2 * 2; };
     const char *xt = reinterpret_cast<const char *>(x + size_t(t0) * G::IN);
     const int xc = lane % G::LPR, xw = wave * G::RPI + lane / G::LPR;  // 16 bytes of a row, row
     unsigned xoff[G::XN];
 #pragma unroll
     for (int m = 0; m < G::XN; ++m)
-        xoff[m] = unsigned(min(m * G::NW * G::RPI + xw, T - 1 - t0)) * G::IN * G::EB + 16 * xc;
+        xoff[m] = unsigned(min(min(m * G::NW * G::RPI + xw, G::TT - 1), T - 1 - t0)) * G::IN * G::EB +
+                  16 * xc;
     // The digits of i are walked from a start that differs between neighbouring units: x rows
     // a multiple of 4 KB apart keep one digit's features in one L2 channel, which every
     // workgroup of an XCD would otherwise read at once.
@@ -333,11 +342,11 @@ __device__ __forceinline__ void join_unit(const typename Ops<C.dt>::E *__restric
             }
         };
         // x of a step, global -> registers -> LDS: the features of the waves' chunks at digit i
-        // (features past the last are zero)
+        // (features past the last are zero, and so are whole chunks past the last)
         u32x4 xr[2][G::XN];
         auto chunk_of = [&](int st) { return int(unsigned(st) / G::nI) * G::KW; };
         auto absent = [&](int st) {
-            return G::NJK % 32 != 0 && chunk_of(st) * 32 + xc * (16 / G::EB) >= G::NJK;
+            return G::PAD && chunk_of(st) * 32 + xc * (16 / G::EB) >= G::NJK;
         };
         auto load_x = [&](int st, int set) TRK_INLINE {
             const char *base = xt + (digit(st) * G::NJK + chunk_of(st) * 32) * G::EB;
@@ -348,7 +357,6 @@ __device__ __forceinline__ void join_unit(const typename Ops<C.dt>::E *__restric
         auto store_x = [&](int st, int set, int buf) TRK_INLINE {  // step st's, which load_x read
 #pragma unroll
             for (int m = 0; m < G::XN; ++m) {
-                if (G::TT % (G::NW * G::RPI) != 0 && m * G::NW * G::RPI + xw >= G::TT) continue;
                 E *dst = j2s + put_x[m % G::XPER] + buf * G::KW * G::szX +
                          m / G::XPER * (G::NW * G::RPI * G::XPER / 16) * G::FRAG;
                 const u32x4 v = absent(st) ? u32x4{0, 0, 0, 0} : xr[set][m];
@@ -438,7 +446,7 @@ __device__ __forceinline__ void join_unit(const typename Ops<C.dt>::E *__restric
                 const int f = ch * 32 + 16 * ft + lrow;
                 jn[ft] = f / G::nK;
                 b3[ft] = j3s + (rw * G::nK + f % G::nK) * G::P3K + al * R + cl;
-                if ((G::NJK % 32 != 0 && f >= G::NJK) ||
+                if ((G::PAD && f >= G::NJK) ||
                     (!G::SJ && G::NH == 1 && jn[ft] != jb[ft] + jl))
                     b3[ft] = nullptr;
             }

@@ -273,12 +273,12 @@ def join_geometry(shape: ShapeDecl, order: tuple, t: Tile) -> dict:
     pairs = t.FC * t.SC
     nq, shared = cdiv(pairs, qw), t.KS3 == 1
     slices = t.FC * nj * R * R + t.SC * nk * (R * R + 16)
-    x_chunk = mt * 512 + (0 if shared else 16 // eb)
+    rows = max(1, t.NW * (64 * 16 // (t.KS3 * 32 * eb))) if t.KS3 else 1  # x rows loaded at once
+    x_chunk = rup(t.TT, max(rows, 16)) * 32 + (0 if shared else 16 // eb)
     lds = max(eb * (slices + R * R + 2 * ks * 512 + 2 * t.KS3 * x_chunk),
               min(mt, 4) * 16 * (pairs * 16 + 4) * 4 if shared else t.NW * nq * mt * 1024)
     # registers of the arrays: accumulators, the joined slice and G1's fragments, x read from LDS,
     # two steps of it in flight, a formed tile, and addresses
-    rows = max(1, t.NW * (64 * 16 // (t.KS3 * 32 * eb))) if t.KS3 else 1  # x rows loaded at once
     vgprs = (nq * mt * 4 + (nq * 2 + 1) * ks * 2 * eb + mt * 2 * eb + 9 * cdiv(t.TT, rows)
              + nq * (8 + 2 * eb) + 28)
     g = {"LDS_BYTES": lds, "NBLK": cdiv(q, t.FC) * cdiv(r, t.SC), "TAIL": False,
@@ -294,7 +294,8 @@ def join_geometry(shape: ShapeDecl, order: tuple, t: Tile) -> dict:
         (max(nq, t.SC) % min(nq, t.SC) == 0, "a wave's pairs are whole rows or parts of one"),
         (t.NW in (4, 8) and t.KS3 >= 1 and t.NW % t.KS3 == 0, "KS3 must divide the waves"),
         (t.TT > 0 and t.TT % 16 == 0, "tokens come in tiles of 16"),
-        (cdiv(nj * nk, 32) % t.KS3 == 0, "the waves take equal shares of the chunks"),
+        (t.KS3 < 1 or -cdiv(nj * nk, 32) % t.KS3 * 8 <= rup(cdiv(nj * nk, 32), t.KS3),
+         "at most an eighth of the waves' chunks are empty"),
         (pairs % qw == 0 and t.FC <= q and t.SC <= r, "pairs must split over the waves"),
         (t.NACC in (1, 2) and t.NACC * t.NW <= 8, "at most two waves per SIMD"),
         (lds * t.NACC <= LDS_LIMIT, f"LDS {lds} B exceeds 160 KB per CU"),
