@@ -31,15 +31,17 @@
 // The steps (chunk of 32 features, digit i) run in lockstep over two LDS buffers. Four waves leave
 // a SIMD one wave of up to 512 registers, whose tile amortises formation best (large calls); eight
 // leave it two of half the size, and one issues while the other waits: 5120 -> 12288 R16 T=128 63 ->
-// 59 us, 1920 -> 2880 R16 T=32 9.6 -> 8.0 us, R8 T=1023 31.5 -> 28.8 us.
+// 59 us, 1920 -> 2880 R16 T=32 9.6 -> 8.0 us, R8 T=1023 31.5 -> 29 us.
 //
 // What bounds it: at KW = 1 matrix cores (2-3 times the dense product's work at rank 16: R^2 / TT
 // of formation) and the waits between them; at KW = 4 and 8, where every wave reads its own x and
-// all of G1's fragments, LDS as well. At 14336 -> 4096, rank 16, 256 tokens (94 us) a step's MFMAs
-// take about 770 clocks of a CU and its LDS traffic about 1200: 128 KB of reads at the 206 B/clk
-// measured, 40 KB of writes at 68. Measured against the chains on the same card: 217 -> 94 us
-// there; 5120 -> 12288 R16 T=128 153 -> 59 us; 17408 -> 5120 R16 T=2048 12700 -> 735 us (1.2 PFLOP/s
-// with the formation); 1920 -> 2880 R8 T=1023 51.7 -> 28.8 us, fp32 T=100 41.7 -> 37.5 us.
+// all of G1's fragments, LDS as well. Counters at 14336 -> 4096, rank 16, 256 tokens, when that took
+// 94 us: matrix cores busy 46 % of a CU's clocks, LDS 76 %, a third of that in bank conflicts of x's
+// stores and of the join's reads of G3; with the offsets of x_at, the swap of x_swap and the pad P3K,
+// each of which spreads the 16 lanes that one pass serves, 94 -> 90 us there, 5120 -> 12288 R16
+// T=128 59 -> 55.6 us, 5120 -> 1024 R12 T=300 29.5 -> 27.4 us. Measured against the chains on the same
+// card: 213 -> 90, 151 -> 55.6 and 74.8 -> 27.4 us; 17408 -> 5120 R16 T=2048 12660 -> 730 us (1.2
+// PFLOP/s with the formation); 1920 -> 2880 R8 T=1023 50.7 -> 28.5 us, fp32 T=100 41.7 -> 37.3 us.
 #include "trk_mfma_kernel.h"
 
 namespace trk {
@@ -88,24 +90,29 @@ struct JoinGeo {
     static constexpr int oJ1 = kJoinHeader / EB + R2;
     static constexpr int oJ2 = oJ1 + nI * KS * FRAG;
     static constexpr int oJ3 = oJ2 + oQ * nJ * R2;
-    // LDS, in elements: the workgroup's slices of G2 and G3 (rows of one k 16 elements
-    // past a multiple of the banks), R^2 zeros, two steps of G1's fragments and of x (chunks a
-    // 16-byte unit apart modulo the banks); at the end the partial sums (KW > 1) or 64 tokens of y
+    // LDS, in elements: the workgroup's slices of G2 and G3 (rows of one k 16 bytes past
+    // a multiple of the banks, which 8-byte reads of neighbouring k fill in order; 16-byte reads 32),
+    // R^2 zeros, two steps of G1's fragments and of x; at the end the partial sums (KW > 1) or 64 tokens of y
     // replace them all
-    static constexpr int P3K = R2 + 16;
+    static constexpr int P3K = R2 + (SJ ? 8 : 16);
     static constexpr int szJ2 = FC * nJ * R2, szJ3 = SC * nK * P3K, szG1 = KS * FRAG;
     // one step's x of one chunk: the rows loaded at once are stored without a branch (it would cut
     // the step's schedule in two: 5120 -> 17408 R16 T=160, TT = 160 over 8 waves, 112 -> 106 us), so
     // there is room for those past the tile
     static constexpr int XROWS = XN * NW * RPI > TT ? XN * NW * RPI : TT;
-    static constexpr int szX = XROWS / 16 * FRAG + (KW > 1 ? VPE : 0);
+    // chunk c starts x_at(c) into a step's region: the 16 lanes that one pass of a store serves write
+    // a row of four chunks (KW >= 4), and these offsets give their halves of 16 bytes different banks
+    static constexpr int x_at(int c) {
+        return c * (XROWS / 16 * FRAG) + (EB == 2 ? c % 2 * VPE + c / 2 * 4 * VPE : c * VPE);
+    }
+    static constexpr int szX = KW == 1 ? XROWS / 16 * FRAG : x_at(KW) + VPE;  // one step's x
     static constexpr int lJ3 = szJ2, lZ = lJ3 + szJ3, lG1 = lZ + R2, lX = lG1 + 2 * szG1;
     static constexpr int TILES = NQ * MT, TPW = cdiv(TILES, KW);  // y tiles, per storing wave
     // y through LDS (XS): [token][pair][p], a token's floats 4 words past a multiple of 64
     static constexpr int YG = MT < 4 ? MT : 4, YP = FC * SC * 16 + 4;
     static constexpr int RED_BYTES = KW > 1 ? NW * TILES * 1024 : YG * 16 * YP * 4;
     static constexpr int LDS_BYTES =
-        (lX + 2 * KW * szX) * EB > RED_BYTES ? (lX + 2 * KW * szX) * EB : RED_BYTES;
+        (lX + 2 * szX) * EB > RED_BYTES ? (lX + 2 * szX) * EB : RED_BYTES;
     static constexpr int NBLK = cdiv(oQ, FC) * cdiv(oR, SC);
 
     static_assert(C.F == 1 && C.S == 2 && C.L == 0, "the joined family joins G2 and G3");
@@ -276,10 +283,11 @@ __device__ __forceinline__ void join_unit(const typename Ops<C.dt>::E *__restric
     // 14336 -> 4096 R16 T=256: x then took a third of the time). In 16 bits a lane's 16 bytes are
     // the features of two lane groups of one result; in 32 bits, of one. The lane groups of row w
     // sit at slots g ^ x_swap(w), so that the 32 lanes one LDS pass serves read 32 different
-    // 16-byte units.
+    // 16-byte units, and with shared x (a store's 16 lanes are then four rows, each writing the even or
+    // the odd slots) so that rows two apart write different ones.
     // Byte offsets from the tile's first row (rows past the tile or the last token read the last one;
     // their results are not stored).
-    auto x_swap = [](int row) { return row / 8 % 2 * 2; };
+    auto x_swap = [](int row) { return row / 8 % 2 * 2 + (G::XS && G::EB == 2 ? row / 2 % 2 : 0); };
     const char *xt = reinterpret_cast<const char *>(x + size_t(t0) * G::IN);
     const int xc = lane % G::LPR, xw = wave * G::RPI + lane / G::LPR;  // 16 bytes of a row, row
     unsigned xoff[G::XN];
@@ -297,7 +305,7 @@ __device__ __forceinline__ void join_unit(const typename Ops<C.dt>::E *__restric
     // fragment reads: one address register per region, everything else in the instruction's
     // offset field (the regions start past its 64 KB)
     int lane_g1 = G::lG1 + lane * G::VPE;
-    int lane_x = G::lX + kw * G::szX + (lrow * 4 + (lgrp ^ x_swap(lrow))) * G::VPE;
+    int lane_x = G::lX + G::x_at(kw) + (lrow * 4 + (lgrp ^ x_swap(lrow))) * G::VPE;
     int put_x[G::XPER];
 #pragma unroll
     for (int m = 0; m < G::XPER; ++m) {
@@ -305,12 +313,14 @@ __device__ __forceinline__ void join_unit(const typename Ops<C.dt>::E *__restric
         // (16 bits: groups 2 (s % 2) and the next, result s / 2, which x_swap leaves neighbours)
         constexpr int SPC = G::LPR / G::KW;  // lanes of a row per chunk
         const int sl = xc % SPC;
-        put_x[m] = G::lX + xc / SPC * G::szX + row / 16 * G::FRAG + w * 4 * G::VPE +
+        put_x[m] = G::lX + G::x_at(xc / SPC) + row / 16 * G::FRAG + w * 4 * G::VPE +
                    (G::EB == 2 ? ((2 * (sl % 2)) ^ x_swap(w)) * 8 + sl / 2 * 4
                                : sl / 4 * 256 + (sl % 4 ^ x_swap(w)) * 4);
         asm("" : "+v"(put_x[m]));
     }
-    asm("" : "+v"(lane_g1), "+v"(lane_x));
+    // (shared x: where a row's odd lane groups go, on the side of the even ones that x_swap says)
+    int put_x2 = put_x[0] + (x_swap(xw % 16) % 2 ? -8 : 8);
+    asm("" : "+v"(lane_g1), "+v"(lane_x), "+v"(put_x2));
 
     f32x4 gate[PAIR ? G::TPW : 1];
 #pragma unroll 1
@@ -357,12 +367,14 @@ __device__ __forceinline__ void join_unit(const typename Ops<C.dt>::E *__restric
         auto store_x = [&](int st, int set, int buf) TRK_INLINE {  // step st's, which load_x read
 #pragma unroll
             for (int m = 0; m < G::XN; ++m) {
-                E *dst = j2s + put_x[m % G::XPER] + buf * G::KW * G::szX +
+                E *dst = j2s + put_x[m % G::XPER] + buf * G::szX +
                          m / G::XPER * (G::NW * G::RPI * G::XPER / 16) * G::FRAG;
                 const u32x4 v = absent(st) ? u32x4{0, 0, 0, 0} : xr[set][m];
                 if constexpr (G::EB == 2) {
                     *reinterpret_cast<u32x2 *>(dst) = u32x2{v[0], v[1]};
-                    *reinterpret_cast<u32x2 *>(dst + 8) = u32x2{v[2], v[3]};
+                    E *dst2 = G::XS ? j2s + put_x2 + buf * G::szX + m * (G::NW * G::RPI / 16) * G::FRAG
+                                    : dst + 8;
+                    *reinterpret_cast<u32x2 *>(dst2) = u32x2{v[2], v[3]};
                 } else {
                     *reinterpret_cast<u32x4 *>(dst) = v;
                 }
@@ -501,7 +513,7 @@ __device__ __forceinline__ void join_unit(const typename Ops<C.dt>::E *__restric
             V8 xl[G::MT];
 #pragma unroll
             for (int m = 0; m < G::MT; ++m)
-                xl[m] = join_read<O>(j2s + lane_x + P * G::KW * G::szX + m * G::FRAG);
+                xl[m] = join_read<O>(j2s + lane_x + P * G::szX + m * G::FRAG);
             Acc<32> w[G::NQ][2];
 #pragma unroll
             for (int n = 0; n < G::NQ; ++n)

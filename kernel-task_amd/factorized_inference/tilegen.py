@@ -272,10 +272,12 @@ def join_geometry(shape: ShapeDecl, order: tuple, t: Tile) -> dict:
     qw = t.NW // t.KS3 if t.KS3 and t.NW % t.KS3 == 0 else 1
     pairs = t.FC * t.SC
     nq, shared = cdiv(pairs, qw), t.KS3 == 1
-    slices = t.FC * nj * R * R + t.SC * nk * (R * R + 16)
+    slices = t.FC * nj * R * R + t.SC * nk * (R * R + (8 if nk % 16 == 0 else 16))
     rows = max(1, t.NW * (64 * 16 // (t.KS3 * 32 * eb))) if t.KS3 else 1  # x rows loaded at once
-    x_chunk = rup(t.TT, max(rows, 16)) * 32 + (0 if shared else 16 // eb)
-    lds = max(eb * (slices + R * R + 2 * ks * 512 + 2 * t.KS3 * x_chunk),
+    vpe = 16 // eb
+    skew = t.KS3 % 2 * vpe + t.KS3 // 2 * 4 * vpe if eb == 2 else t.KS3 * vpe
+    x_step = t.KS3 * rup(t.TT, max(rows, 16)) * 32 + (0 if shared else skew + vpe)
+    lds = max(eb * (slices + R * R + 2 * ks * 512 + 2 * x_step),
               min(mt, 4) * 16 * (pairs * 16 + 4) * 4 if shared else t.NW * nq * mt * 1024)
     # registers of the arrays: accumulators, the joined slice and G1's fragments, x read from LDS,
     # two steps of it in flight, a formed tile, and addresses
