@@ -12,7 +12,8 @@
  *     trk_last_error() returns the message of the last failure on the calling thread.
  *   - Core k is [R][o_k][i_k][R] row-major; x is [T][in] row-major; y is [T][out] row-major,
  *     with in = (i*nj + j)*nk + k and out = (p*Q + q)*Rr + r. All three share one dtype.
- *   - A plan is immutable after trk_plan_create (trk_plan_set_variant aside), so one plan
+ *   - A plan is immutable after trk_plan_create (trk_plan_set_variant and trk_plan_admit aside),
+ *     so one plan
  *     may be used from several host threads and streams at once: trk_forward keeps no state
  *     between calls, allocates nothing and needs no workspace.
  *
@@ -147,6 +148,16 @@ int trk_plan_set_variant(trk_plan *plan, int t_min, int t_max, int variant);
  * on `stream`. The cores are only read. Replaces pack_cores (tr_kernel.py:86-99). */
 int trk_pack(const trk_plan *plan, const void *g1, const void *g2, const void *g3,
              void *packed, void *stream);
+
+/* Let the plan's default selection use its fp16 joined-core variants for the cores packed in
+ * `packed`: waits on `stream` for their packing and reads what it found. Those variants form
+ * products of two and three cores in fp16, which keep the other variants' precision only where
+ * the values of each core are of one size; until this call, and for good where a packed buffer's
+ * cores are not, the selection keeps to the variants that round sums of x alone. A plan used with
+ * several packed buffers is shown each of them. Does nothing, and does not wait, for plans of other
+ * dtypes; an explicit variant index and trk_plan_set_variant are not bound by it. Not thread-safe
+ * against other calls on the same plan. No reference counterpart. */
+int trk_plan_admit(trk_plan *plan, const void *packed, void *stream);
 
 /* y = TR(cores) x for `tokens` rows of x, on `stream`, with the variant the plan selects.
  * x and packed are only read; y is fully written; tokens == 0 launches nothing. x and packed

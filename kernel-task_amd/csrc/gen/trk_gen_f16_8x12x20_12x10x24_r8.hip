@@ -13,8 +13,7 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape210, 1, 1, 10, 12, 8, 2, 1, 8, 32, 8), 3, 8)  // wide8x32w8_t1k2n1_ic8
     TRK_ENTRY(tile(kShape210, 1, 1, 10, 12, 4, 2, 1, 4, 32, 4, 0, 0, 0, 0, 1), 9, 32)  // wide4x32_t1k2n1_ic4_sl
     TRK_ENTRY(tile(kShape210, 1, 2, 10, 12, 4, 2, 1, 4, 32, 4, 0, 0, 0, 0, 1), 33, 64)  // ring3_mfma_wide4x32_sl<210,1,2,10,12,4,2,1>
-    TRK_ENTRY(tile(kShape210, 1, 8, 10, 12, 2, 1, 2, 4, 32, 8, 1), 65, 80)  // ring3_mfma_wide4x32w8p<210,1,8,10,12,2,1,2>
-    TRK_ENTRY(tile(kShape210, 1, 8, 10, 12, 2, 1, 2, 4, 32, 8, 1), 129, 160)  // ring3_mfma_wide4x32w8p<210,1,8,10,12,2,1,2>
+    TRK_ENTRY(tile(kShape210, 1, 8, 10, 12, 2, 1, 2, 4, 32, 8, 1), 65, 1073741824)  // ring3_mfma_wide4x32w8p<210,1,8,10,12,2,1,2>
     TRK_ENTRY(tile(kShape210, 1, 1, 10, 12, 8, 4, 1, 0, 16, 8, 0, 0, 1), 0, 0)  // t1_all_w8_xl
     TRK_ENTRY(tile(kShape210, 3, 1, 10, 12, 4, 2, 1, 4, 32, 4), 0, 0)  // cover_t3_w4
     TRK_ENTRY(tile(kShape210, 2, 3, 10, 12, 2, 2, 1, 4, 32, 4), 0, 0)  // cover_t2f3_w4

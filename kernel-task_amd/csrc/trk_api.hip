@@ -50,6 +50,36 @@ void grid_of(const Plan &p, const Variant &v, int tokens, int grid[3]) {
         grid[2] = 1;
     }
 }
+
+// The variant of a call: later entries were registered for narrower token ranges (the joined-core
+// ones last) and win over earlier ones; gated ones count where the plan is admitted.
+int select_variant(const Plan &p, int tokens, bool admitted) {
+    for (int i = p.nvariants - 1; i > 0; --i) {
+        const Variant &v = p.variants[i];
+        if (v.t_min > 0 && tokens >= v.t_min && tokens <= v.t_max && (admitted || !v.gated)) return i;
+    }
+    return 0;
+}
+
+// The token range the default selection routes to variant i (0, 0: none): the range it holds, for
+// a gated variant of a plan that is not admitted none, and for the chain variants under admitted
+// gated ones without what those take at its ends.
+void routed_range(const Plan &p, int i, int *t_min, int *t_max) {
+    int lo = p.variants[i].t_min, hi = p.variants[i].t_max;
+    if (p.variants[i].gated && p.admitted <= 0) lo = hi = 0;
+    bool moved = p.admitted > 0 && !p.variants[i].gated && p.variants[i].kind == TRK_KERNEL_MFMA;
+    while (moved && lo > 0 && lo <= hi) {
+        moved = false;
+        for (int k = i + 1; k < p.nvariants; ++k) {
+            const Variant &w = p.variants[k];
+            if (!w.gated || w.t_min <= 0) continue;
+            if (w.t_min <= lo && lo <= w.t_max) lo = w.t_max + 1, moved = true;
+            if (w.t_min <= hi && hi <= w.t_max) hi = w.t_min - 1, moved = true;
+        }
+    }
+    *t_min = lo <= hi ? lo : 0;
+    *t_max = lo <= hi ? hi : 0;
+}
 }  // namespace
 
 // Index of the chain with this order and these K-order groups in the plan, adding it (and
@@ -274,13 +304,7 @@ size_t trk_plan_packed_bytes(const trk_plan *plan) {
 int trk_plan_variant_count(const trk_plan *plan) { return plan ? as_plan(plan)->nvariants : 0; }
 
 int trk_plan_select(const trk_plan *plan, int tokens) {
-    if (!plan) return -1;
-    const Plan &p = *as_plan(plan);
-    // later entries were registered for narrower token ranges and win over earlier ones
-    for (int i = p.nvariants - 1; i > 0; --i)
-        if (tokens >= p.variants[i].t_min && tokens <= p.variants[i].t_max && p.variants[i].t_min > 0)
-            return i;
-    return 0;
+    return plan ? select_variant(*as_plan(plan), tokens, as_plan(plan)->admitted > 0) : -1;
 }
 
 int trk_plan_describe(const trk_plan *plan, int variant, int tokens, trk_variant_info *info) {
@@ -300,8 +324,7 @@ int trk_plan_describe(const trk_plan *plan, int variant, int tokens, trk_variant
     grid_of(p, v, tokens, info->grid);
     info->block = v.block;
     info->lds_bytes = v.lds_bytes;
-    info->t_min = v.t_min;
-    info->t_max = v.t_max;
+    routed_range(p, variant, &info->t_min, &info->t_max);
     // algorithmic work of the cores' rank (a padded plan's kernels do more, on zeros)
     info->flops = chain_flops_per_token(p, c, p.core_rank) * tokens;
     double params = 0.0;
@@ -337,6 +360,27 @@ int trk_plan_set_variant(trk_plan *plan, int t_min, int t_max, int variant) {
     if (variant > 0) {
         p.variants[variant].t_min = t_min;
         p.variants[variant].t_max = t_max;
+        p.variants[variant].gated = 0;  // the caller's choice
+    }
+    return TRK_OK;
+}
+
+int trk_plan_admit(trk_plan *plan, const void *packed, void *stream) {
+    if (!plan || !packed) return set_error(TRK_ERR_INVALID, "trk_plan_admit: null argument");
+    Plan &p = *as_plan(plan);
+    if (p.dtype != TRK_DTYPE_F16 || p.admitted < 0) return TRK_OK;
+    for (int i = 0; i < p.nchains; ++i) {
+        if (!p.chains[i].join) continue;
+        unsigned uneven = 1;
+        const char *verdict = static_cast<const char *>(packed) + p.chains[i].offF + 4 * kJoinUneven;
+        int st = check_hip(hipMemcpyAsync(&uneven, verdict, sizeof(uneven), hipMemcpyDeviceToHost,
+                                          static_cast<hipStream_t>(stream)),
+                           "trk_plan_admit: copy");
+        if (st == TRK_OK)
+            st = check_hip(hipStreamSynchronize(static_cast<hipStream_t>(stream)),
+                           "trk_plan_admit: wait");
+        if (st != TRK_OK) return st;
+        p.admitted = uneven ? -1 : 1;
     }
     return TRK_OK;
 }
@@ -407,10 +451,7 @@ int trk_forward_swiglu(const trk_plan *gate, const void *packed_gate, const trk_
                          "trk_forward_swiglu: the gate and up plans differ in shape, dtype, rank "
                          "or packed layout");
     if (tokens == 0) return TRK_OK;
-    const int variant = trk_plan_select(gate, tokens);
-    if (variant < 0 || variant >= g.nvariants)
-        return set_error(TRK_ERR_INVALID, "trk_forward_swiglu: no variant for %d tokens", tokens);
-    const Variant &v = g.variants[variant];
+    const Variant &v = g.variants[select_variant(g, tokens, g.admitted > 0 && u.admitted > 0)];
     const Chain &cg = g.chains[v.chain], &cu = u.chains[v.chain];
     if (cg.offF != cu.offF || cg.offS != cu.offS || cg.offL != cu.offL)
         return set_error(TRK_ERR_INVALID, "trk_forward_swiglu: the plans' packed layouts differ");

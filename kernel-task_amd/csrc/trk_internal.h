@@ -68,6 +68,7 @@ struct Variant {
     int block;       // threads per workgroup
     int lds_bytes;   // dynamic LDS per workgroup
     int t_min, t_max;
+    int gated;       // 1: the default selection routes here once the plan is admitted
     int xcd_local;   // XCDs the launch's work runs on: 0 = all 8; 1, 2, 4 (KCfg::XL; grid x 8/XL)
     char name[64];
     LaunchFn launch;
@@ -83,6 +84,7 @@ struct Plan {
     int nvariants;
     Variant variants[kMaxVariants];
     size_t packed_bytes;
+    int admitted;  // gated variants: 0 not yet (trk_plan_admit), 1 routed, -1 refused for good
 };
 
 // error reporting (trk_api.hip)
@@ -96,9 +98,10 @@ void describe_chain(const int in_modes[3], const int out_modes[3], int rank, con
 int plan_chain(Plan *plan, const int order[3], int sg, int lg, int sfrag);
 // index of the plan's joined-core section, added if new (-1: full)
 int plan_join_chain(Plan *plan);
-// The joined-core section: kJoinHeader bytes whose first float is the factor of the results,
-// R^2 zeros, then J1, J2 and J3 (trk_pack.hip).
-constexpr int kJoinHeader = 256;
+// The joined-core section: kJoinHeader bytes whose first float is the factor of the results and
+// whose word kJoinUneven is nonzero for fp16 cores too uneven for one scale each, R^2 zeros, then
+// J1, J2 and J3 (trk_pack.hip).
+constexpr int kJoinHeader = 256, kJoinUneven = 63;
 
 // Entry points a variant module (a generated table built at prepare time) exports, and the
 // layout check its loader applies: the module's sizeof(Plan) must equal the library's.

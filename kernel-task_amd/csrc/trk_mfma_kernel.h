@@ -1600,6 +1600,7 @@ inline int register_entries(Plan *plan, const Entry *entries, int count) {
         v.t_max = e.t_max;
         v.launch = e.launch;
         v.launch_pair = e.launch_pair;
+        v.gated = k.JN && k.dt == TRK_DTYPE_F16;  // its 16-bit intermediates need even cores
         v.xcd_local = k.XL;
         if (k.JN) {
             std::snprintf(v.name, sizeof(v.name), "ring3_join%s<%d%d%d,%d,%d,%d,%d,%d,%d,%d>",

@@ -148,14 +148,16 @@ int pack_all(const Plan &plan, const void *const g[3], void *packed, hipStream_t
 // subnormal), and the header's first float is the factor that undoes it on the fp32 sums:
 // products of two and three cores are formed in the cores' type, and cores far from 1 would leave
 // fp16's range there. The header's next 3 x kPeaks floats are the largest magnitudes of the
-// cores' parts (infinite where a part holds an infinity or a NaN). bf16 and fp32 have the range.
+// cores' parts (infinite where a part holds an infinity or a NaN), and the word kJoinUneven says
+// whether a core is too uneven for one scale (join_spread_kernel). bf16 and fp32 have the range.
 struct JoinArgs {
     int R, Rc, nI, nJ, nK, oP, oQ, oR;
     unsigned nJ1, nJ2, nJ3;  // (plan_join_chain keeps the section below 2^31 elements)
 };
 
 constexpr int kPeaks = 16;  // workgroups per core that look for its largest magnitude
-static_assert((1 + 3 * kPeaks) * 4 <= kJoinHeader, "the peaks fit the header");
+static_assert(1 + 3 * kPeaks <= kJoinUneven && (kJoinUneven + 1) * 4 <= kJoinHeader,
+              "the peaks and the verdict fit the header");
 
 template <int DT>
 __global__ void __launch_bounds__(1024) join_peak_kernel(
@@ -177,15 +179,78 @@ __global__ void __launch_bounds__(1024) join_peak_kernel(
         __syncthreads();
     }
     if (threadIdx.x == 0) peaks[blockIdx.y * kPeaks + blockIdx.x] = part[0];
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0)  // join_spread_kernel may raise it
+        reinterpret_cast<unsigned *>(peaks - 1)[kJoinUneven] = 0;
+}
+
+__device__ inline float join_peak(const float *peaks) {
+    float m = 0.0f;
+    for (int i = 0; i < kPeaks; ++i) m = fmaxf(m, peaks[i]);
+    return m;
 }
 
 // The power of two just above the largest of a core's peaks (0 if that is 0 or not finite).
 __device__ inline int join_exponent(const float *peaks) {
-    float m = 0.0f;
-    for (int i = 0; i < kPeaks; ++i) m = fmaxf(m, peaks[i]);
+    const float m = join_peak(peaks);
     int e = 0;
     if (m > 0.0f && m <= 3.4028234e38f) frexpf(m, &e);
     return e;
+}
+
+// Whether one scale per core keeps the joined kernel's fp16 intermediates (products of two and of
+// three scaled cores) out of fp16's subnormals, where they would lose bits that the chains, which
+// round only sums that x is part of, keep. One workgroup looks at one slice (one index of one of a
+// core's four modes). The core is uneven if the mean magnitude of a slice's nonzero values is
+// below 1/16 of the core's peak, or more than a quarter of them lie below 1/64 of it. Values of
+// an even core then average 2^-5 at least after the scaling, H 2^-8.5 and W 2^-10 at rank 8 (the
+// fewest terms): 4 bits above the subnormals. Normal, uniform and Laplace values pass (means of
+// 1/6, 1/2 and 1/12 of the peak of 10^5 values), digits whose sizes differ by 3 in all three cores
+// just so. In a model of both kernels' roundings every set of cores that passes has the
+// chains' error (2.9e-4), and the first to lose a tenth more is far past the bound.
+constexpr float kJoinMean = 16.0f, kJoinSmall = 64.0f;
+constexpr unsigned kJoinSmallShare = 4;
+
+__global__ void __launch_bounds__(256) join_spread_kernel(const _Float16 *__restrict__ g1,
+                                                          const _Float16 *__restrict__ g2,
+                                                          const _Float16 *__restrict__ g3,
+                                                          float *header, JoinArgs a) {
+    const int k = blockIdx.y;
+    const _Float16 *g = k == 0 ? g1 : k == 1 ? g2 : g3;
+    const unsigned dims[4] = {unsigned(a.Rc), unsigned(k == 0 ? a.oP : k == 1 ? a.oQ : a.oR),
+                              unsigned(k == 0 ? a.nI : k == 1 ? a.nJ : a.nK), unsigned(a.Rc)};
+    unsigned slice = blockIdx.x, mode = 0;
+    while (mode < 4 && slice >= dims[mode]) slice -= dims[mode++];
+    if (mode == 4) return;  // (the grid is as wide as the core with the most slices)
+    unsigned inner = 1, all = dims[0] * dims[1] * dims[2] * dims[3];
+    for (unsigned m = mode + 1; m < 4; ++m) inner *= dims[m];
+    const unsigned n = all / dims[mode];
+    const float peak = join_peak(header + 1 + k * kPeaks);
+    float sum = 0.0f;
+    unsigned nonzero = 0, small = 0;
+    for (unsigned e = threadIdx.x; e < n; e += 256) {
+        const float v = fabsf(float(g[(e / inner * dims[mode] + slice) * inner + e % inner]));
+        sum += v;
+        nonzero += v != 0.0f;
+        small += v != 0.0f && v * kJoinSmall < peak;
+    }
+    __shared__ float sums[256];
+    __shared__ unsigned counts[256], smalls[256];
+    sums[threadIdx.x] = sum;
+    counts[threadIdx.x] = nonzero;
+    smalls[threadIdx.x] = small;
+    __syncthreads();
+    for (int w = 128; w > 0; w /= 2) {
+        if (threadIdx.x < w) {
+            sums[threadIdx.x] += sums[threadIdx.x + w];
+            counts[threadIdx.x] += counts[threadIdx.x + w];
+            smalls[threadIdx.x] += smalls[threadIdx.x + w];
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0 && counts[0] &&
+        (!(peak <= 3.4028234e38f) || sums[0] * kJoinMean < peak * counts[0] ||
+         smalls[0] * kJoinSmallShare > counts[0]))
+        atomicOr(reinterpret_cast<unsigned *>(header) + kJoinUneven, 1u);
 }
 
 template <int DT>
@@ -246,18 +311,25 @@ int pack_join(const Plan &plan, const Chain &c, const void *const g[3], void *pa
     const unsigned R2 = c.R * c.R;
     const T *t[3] = {static_cast<const T *>(g[0]), static_cast<const T *>(g[1]),
                      static_cast<const T *>(g[2])};
-    if constexpr (DT == TRK_DTYPE_F16) {
-        size_t n[3];
-        for (int k = 0; k < 3; ++k)
-            n[k] = size_t(plan.core_rank) * plan.core_rank * plan.in_modes[k] * plan.out_modes[k];
-        hipLaunchKernelGGL(join_peak_kernel<DT>, dim3(kPeaks, 3), dim3(1024), 0, stream, t[0], t[1],
-                           t[2], n[0], n[1], n[2], reinterpret_cast<float *>(out) + 1);
-    }
     JoinArgs a{c.R, plan.core_rank,
                plan.in_modes[0], plan.in_modes[1], plan.in_modes[2],
                plan.out_modes[0], plan.out_modes[1], plan.out_modes[2],
                R2 * 16 * plan.in_modes[0], R2 * plan.in_modes[1] * plan.out_modes[1],
                R2 * plan.in_modes[2] * plan.out_modes[2]};
+    if constexpr (DT == TRK_DTYPE_F16) {
+        size_t n[3];
+        for (int k = 0; k < 3; ++k)
+            n[k] = size_t(plan.core_rank) * plan.core_rank * plan.in_modes[k] * plan.out_modes[k];
+        int slices = 0;
+        for (int k = 0; k < 3; ++k)
+            slices = std::max(slices, 2 * plan.core_rank + plan.in_modes[k] + plan.out_modes[k]);
+        float *header = reinterpret_cast<float *>(out);
+        hipLaunchKernelGGL(join_peak_kernel<DT>, dim3(kPeaks, 3), dim3(1024), 0, stream, t[0], t[1],
+                           t[2], n[0], n[1], n[2], header + 1);
+        hipLaunchKernelGGL(join_spread_kernel, dim3(slices, 3), dim3(256), 0, stream,
+                           static_cast<const _Float16 *>(g[0]), static_cast<const _Float16 *>(g[1]),
+                           static_cast<const _Float16 *>(g[2]), header, a);
+    }
     const unsigned total = R2 + a.nJ1 + a.nJ2 + a.nJ3;
     hipLaunchKernelGGL(join_pack_kernel<DT>, dim3(std::min(total / 256 + 1, 4096u)), dim3(256), 0,
                        stream, t[0], t[1], t[2], out, a);

@@ -65,6 +65,7 @@ SIGNATURES = {
     "trk_plan_describe": (_c_int, [_c_void_p, _c_int, _c_int, ctypes.POINTER(VariantInfo)]),
     "trk_plan_set_variant": (_c_int, [_c_void_p, _c_int, _c_int, _c_int]),
     "trk_pack": (_c_int, [_c_void_p] * 6),
+    "trk_plan_admit": (_c_int, [_c_void_p] * 3),
     "trk_forward": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p]),
     "trk_forward_variant": (_c_int, [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int,
                                      _c_void_p]),

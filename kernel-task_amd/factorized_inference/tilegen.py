@@ -794,10 +794,12 @@ def add_candidate(cands: dict, name: str, order: tuple, tile: Tile) -> str | Non
 
 
 def table(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = False,
-          extended: bool = False) -> list[tuple[str, tuple, Tile, int, int]]:
+          extended: bool = False, admitted: bool = False) -> list[tuple[str, tuple, Tile, int, int]]:
     """[(name, order, tile, t_min, t_max)] for one shape: the tuned winners when the shape
     has measurements, else every candidate with the rule's ranges (0, 0: index only).
-    A tuned entry's "ranges" are its chain tiles, "joined" its joined-core tiles. Its "extra"
+    A tuned entry's "ranges" are its chain tiles, "joined" its joined-core tiles. In fp16 the
+    chains' ranges cover every token count and the joined tiles' lie over them, for plans whose
+    cores trk_plan_admit finds even; they are 0, 0 here unless `admitted` asks for them. Its "extra"
     tiles are compiled index-only beside the winners (alternatives a caller may route token
     counts to, such as the XCD-local tiles).
     all_candidates=True ignores the measurements (the autotuner's input)."""
@@ -806,6 +808,8 @@ def table(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = Fa
     if entry:
         rows = [(r["name"], tuple(r.get("order", entry["order"])), Tile(**r["tile"]),
                  r["t_min"], r["t_max"]) for r in entry["ranges"] + entry.get("joined", [])]
+        if shape.dtype == "f16" and not admitted:
+            rows = [(n, o, t, 0, 0) if t.JN else (n, o, t, lo, hi) for n, o, t, lo, hi in rows]
         rows += [(r["name"], tuple(r.get("order", entry["order"])), Tile(**r["tile"]), 0, 0)
                  for r in entry.get("extra", [])]
         for name, order, t, _, _ in rows:
@@ -860,7 +864,8 @@ def emit(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = Fal
     """One translation unit: the shape's chain tiles, or (join) its joined-core tiles, which
     build_ext compiles with other flags."""
     tuned = load_tuned() if tuned is None else tuned
-    rows = [r for r in table(shape, tuned, all_candidates, extended) if bool(r[2].JN) == join]
+    rows = [r for r in table(shape, tuned, all_candidates, extended, admitted=True)
+            if bool(r[2].JN) == join]
     orders = sorted({r[1] for r in rows}, key=lambda od: (od != choose_order(shape), od))
     i, o = shape.ins, shape.outs
     tuned_note = ("token ranges measured by kernel-task_amd/benchmarks/autotune.py"

@@ -143,9 +143,11 @@ class PreparedTRKernel(_CallBase):
         with torch.cuda.device(self.device_index):
             self.packed = torch.empty(self.plan.packed_bytes, dtype=torch.uint8, device=device)
             g = [c.contiguous() for c in cores]
-            _lib.check(_lib.load().trk_pack(self.plan.handle, g[0].data_ptr(), g[1].data_ptr(),
-                                            g[2].data_ptr(), self.packed.data_ptr(),
-                                            current_stream_handle(self.device_index)))
+            lib, stream = _lib.load(), current_stream_handle(self.device_index)
+            _lib.check(lib.trk_pack(self.plan.handle, g[0].data_ptr(), g[1].data_ptr(),
+                                    g[2].data_ptr(), self.packed.data_ptr(), stream))
+            # fp16: joined-core variants for cores whose values are of one size
+            _lib.check(lib.trk_plan_admit(self.plan.handle, self.packed.data_ptr(), stream))
             # the packed cores are complete before prepare returns, so a first call on any
             # stream (not only the one that packed) reads them whole
             torch.cuda.current_stream(self.device_index).synchronize()

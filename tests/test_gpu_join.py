@@ -11,6 +11,7 @@ import torch
 
 from factorized_inference import TRSpec, _lib, make_cores, prepare_optimized
 from factorized_inference.tr_kernel import current_stream_handle, forward_swiglu
+import join_model as jm
 from gpu_util import check_result, oracle_y
 from oracle import ring_oracle as orc
 
@@ -118,6 +119,25 @@ def test_fp16_cores_far_from_one(scales):
         y = run.run_variant(x, index, _lib.EPI_F32)[:4].double().cpu().numpy()
         # (the cores' own subnormal values carry fewer bits, in the oracle alike)
         assert np.linalg.norm(y - expected) <= 2.0 ** -10 * norm, info["name"]
+
+
+@pytest.mark.parametrize("rank", [8, 16])
+@pytest.mark.parametrize("name", jm.CASES)
+def test_fp16_calls_are_exact_for_uneven_cores(name, rank):
+    # joined tiles form products of two and three cores in fp16: cores whose slices differ in size
+    # keep the chains, and every call is as close to the 64-bit result as below the joined counts
+    x, cores = jm.make(name, rank, 201)
+    spec = TRSpec(jm.INS, jm.OUTS, rank)
+    run = prepare_optimized([c.cuda() for c in cores], spec)
+    assert ("join" in run.selected(201)["name"]) == jm.even(cores), name
+    assert "join" not in run.selected(8)["name"]
+    rows = [0, 99, 200]
+    want = oracle_y(x[rows], cores, spec)
+    got = run.accumulate(x.cuda())[rows].double().cpu().numpy()
+    small = run.accumulate(x[:8].cuda())[:1].double().cpu().numpy()
+    # two roundings of intermediates, as REL; each output digit's share of them is of its own size
+    for y, e in ((got, want), (small, want[:1])):
+        assert np.linalg.norm(y - e) <= REL[torch.float16] * np.linalg.norm(e), name
 
 
 def test_swiglu_pair_of_joined_tiles():
