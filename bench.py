@@ -145,7 +145,7 @@ def measure_case(label, ins, outs, rank, dtype_name, init, tokens, steps, warmup
         max_ref = ref.abs().max().item()
         del y, yf, ref, diff
         info = run.selected(T)
-        flops = m.launch_flops(info, spec, T)
+        flops = run.plan.launch_flops(tokens=T)
         ref_flops = m.reference_flops(spec, T)
         peak = m.PEAK_TFLOPS[dtype]
         case = {

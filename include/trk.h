@@ -77,7 +77,8 @@ typedef struct trk_variant_info {
     int lds_bytes;  /* LDS per workgroup */
     int t_min;      /* smallest token count the default selection routes here (0 = none) */
     int t_max;      /* largest token count the default selection routes here */
-    double flops;   /* algorithmic flops of one launch at that token count, no padding */
+    double flops;   /* flops of taking that many tokens through the cores in `order`, no padding:
+                       what a launch of a chain variant runs (trk_plan_launch_flops: any variant) */
     double bytes;   /* compulsory HBM bytes of one launch: cores + x + y */
     size_t packed_offset[3]; /* byte offsets in the packed buffer of the first, second and
                                 last core as this variant's kernel reads them */
@@ -138,6 +139,12 @@ int trk_plan_select(const trk_plan *plan, int tokens);
  * Replaces the queries smem_bytes / y_tiles / max_y_tiles (tr_ring.cu:363-372) and
  * v3t_smem (tr_ring.cu:1143-1151). */
 int trk_plan_describe(const trk_plan *plan, int variant, int tokens, trk_variant_info *info);
+
+/* Algorithmic flops, without padding, of one launch of `variant` (-1 = the one selected for
+ * `tokens`): for the chain variants trk_variant_info.flops, for the joined-core ones
+ * 2 * (in * out * (tokens + R^2) + nj * nk * q * r * R^3), the second and third cores joined, the
+ * first with the result, each once, and x with that. No reference counterpart. */
+int trk_plan_launch_flops(const trk_plan *plan, int variant, int tokens, double *flops);
 
 /* Route token counts in [t_min, t_max] to `variant` from now on (tuning and tests). Replaces
  * the TR_KC / TR_TT / TR_QC / TR_V3T_TILING overrides read by tr_kernel.py:118-176,

@@ -240,7 +240,8 @@ def measure(case: Case) -> dict:
     if prepared is not None:
         info = prepared.selected(case.tokens)
         kernel = {"variant": info["name"], "grid": info["grid"], "lds_bytes": info["lds_bytes"],
-                  "packed_bytes": prepared.packed_bytes, "flops": info["flops"],
+                  "packed_bytes": prepared.packed_bytes,
+                  "flops": prepared.plan.launch_flops(tokens=case.tokens),
                   "compulsory_bytes": info["bytes"]}
     return {
         **result, "preparation_ms": prep_ms, "first_call_ms": first_ms,

@@ -192,7 +192,7 @@ def cases(trace: Path, details: dict, max_gap_us: float = 30.0) -> list[dict]:
     """Per bench.py case (details["cases"], from the traced run): the kernel of its variant at
     its grid in the trace, with dispatches, mean / min / median duration and the longest
     back-to-back block (grids()), the case's stream time in the same run, and the roofline
-    fractions of the trace mean (algorithmic bytes / 8 TB/s, chain-order flops / peak)."""
+    fractions of the trace mean (algorithmic bytes / 8 TB/s, flops of the launch / peak)."""
     import dataclasses
 
     sys.path.insert(0, str(Path(__file__).resolve().parents[1]))

@@ -13,7 +13,7 @@ seed 0, harness protocol): per shape, rank and token count, the HIP-event stream
 the prepared operator (the generated, autotuned MFMA tables) and of F.linear on the
 materialised weight, timed the same way in one process, with the relative L2 error of
 both against an fp64 dense product on a subset of token rows, and the algorithmic rates
-(flops of the contraction order the kernel runs, compulsory bytes).
+(flops of the contraction the kernel runs, compulsory bytes).
 """
 from __future__ import annotations
 
@@ -34,7 +34,6 @@ import torch  # noqa: E402
 from factorized_inference import (  # noqa: E402
     TRSpec, dense_forward, make_cores, materialize_dense_weight, prepare_optimized, tilegen,
 )
-from factorized_inference.measure import launch_flops  # noqa: E402
 
 PEAK_TFLOPS, PEAK_GBS = 2500.0, 8000.0
 
@@ -106,7 +105,7 @@ def main() -> int:
                 sub = x[: min(T, 8)]
                 ref = sub.double() @ w64.T
                 info = run.selected(T)
-                flops = launch_flops(info, spec, T)
+                flops = run.plan.launch_flops(tokens=T)
                 row = {"shape": shape.name, "key": shape.key, "rank": shape.rank, "tokens": T,
                        "dtype": args.dtype, "kernel_rank": run.plan.kernel_rank,
                        "modules": run.plan.modules, "kind": info["kind"],

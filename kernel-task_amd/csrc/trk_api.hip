@@ -337,6 +337,22 @@ int trk_plan_describe(const trk_plan *plan, int variant, int tokens, trk_variant
     return TRK_OK;
 }
 
+int trk_plan_launch_flops(const trk_plan *plan, int variant, int tokens, double *flops) {
+    if (!plan || !flops) return set_error(TRK_ERR_INVALID, "trk_plan_launch_flops: null argument");
+    const Plan &p = *as_plan(plan);
+    if (tokens < 0) return set_error(TRK_ERR_INVALID, "trk_plan_launch_flops: tokens < 0");
+    if (variant < 0) variant = trk_plan_select(plan, tokens);
+    if (variant >= p.nvariants)
+        return set_error(TRK_ERR_INVALID, "trk_plan_launch_flops: no variant %d", variant);
+    const Chain &c = p.chains[p.variants[variant].chain];
+    const double R = p.core_rank;
+    *flops = !c.join    ? chain_flops_per_token(p, c, p.core_rank) * tokens
+             : !tokens ? 0.0
+                        : 2.0 * (double(p.in_features) * p.out_features * (tokens + R * R) +
+                                 double(c.nF) * c.oF * c.nS * c.oS * R * R * R);
+    return TRK_OK;
+}
+
 int trk_plan_set_variant(trk_plan *plan, int t_min, int t_max, int variant) {
     if (!plan) return set_error(TRK_ERR_INVALID, "trk_plan_set_variant: null plan");
     Plan &p = *as_plan(plan);

@@ -63,6 +63,7 @@ SIGNATURES = {
     "trk_plan_variant_count": (_c_int, [_c_void_p]),
     "trk_plan_select": (_c_int, [_c_void_p, _c_int]),
     "trk_plan_describe": (_c_int, [_c_void_p, _c_int, _c_int, ctypes.POINTER(VariantInfo)]),
+    "trk_plan_launch_flops": (_c_int, [_c_void_p, _c_int, _c_int, ctypes.POINTER(ctypes.c_double)]),
     "trk_plan_set_variant": (_c_int, [_c_void_p, _c_int, _c_int, _c_int]),
     "trk_pack": (_c_int, [_c_void_p] * 6),
     "trk_plan_admit": (_c_int, [_c_void_p] * 3),
@@ -153,6 +154,12 @@ class Plan:
         check(self._lib.trk_plan_describe(self.handle, int(variant), int(tokens),
                                           ctypes.byref(info)))
         return info.as_dict()
+
+    def launch_flops(self, variant: int = -1, tokens: int = 1) -> float:
+        flops = ctypes.c_double()
+        check(self._lib.trk_plan_launch_flops(self.handle, int(variant), int(tokens),
+                                              ctypes.byref(flops)))
+        return flops.value
 
     def variants(self, tokens: int = 1) -> list[dict]:
         return [self.describe(v, tokens) for v in range(self.variant_count)]

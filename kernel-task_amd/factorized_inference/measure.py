@@ -140,18 +140,6 @@ def reference_flops(spec, tokens: int) -> float:
     return 2.0 * tokens * per_token
 
 
-def launch_flops(info: dict, spec, tokens: int) -> float:
-    """Algorithmic flops of the kernel a launch runs: the plan's figure (x through the cores in
-    the variant's order) for the chain kernels; for the joined-core ones two cores joined, the
-    third with the result, and x with that, each once."""
-    if "join" not in info["name"]:
-        return info["flops"]
-    R = spec.rank
-    (_, nj, nk), (_, q, r) = spec.input_modes, spec.output_modes
-    return 2.0 * (spec.in_features * spec.out_features * (tokens + R * R)
-                  + nj * nk * q * r * R ** 3)
-
-
 def floors(lib, calls: int = 2000) -> dict:
     """Host cost of an empty C call and of an empty launch; stream time of empty launches
     (the reference's floors, tools/measure_kernels.py:97-103, without its profiler kernel

@@ -290,3 +290,26 @@ def test_forward_swiglu_argument_checks():
     for tokens in (1, 2, 5, 33, 200, 4096):
         assert call(g.handle, None, u.handle, None, None, None, tokens, None) == _lib.ERR_INVALID
         assert b"null buffer" in lib.trk_last_error()
+
+
+@pytest.mark.parametrize("rank", [8, 12, 16])
+def test_launch_flops_are_those_of_the_kernel_that_runs(rank):
+    # 5120 -> 12288 (rank 12 on the rank-16 kernels): chains take x through the cores in their
+    # order; joined-core variants join G2 with G3, that with G1, each once, and x with the result
+    ins, outs, tokens = (20, 16, 16), (16, 24, 32), 128
+    plan = _lib.Plan(ins, outs, rank, _lib.DTYPE_BF16, kernel_rank=max(8, 1 << (rank - 1).bit_length()))
+    n_in, n_out = int(np.prod(ins)), int(np.prod(outs))
+    weight = n_in * n_out * rank ** 2 + 16 * 16 * 24 * 32 * rank ** 3
+    kinds = set()
+    for index, v in enumerate(plan.variants(tokens)):
+        joined = "join" in v["name"]
+        kinds.add(joined)
+        chain = orc.flops_per_token(ins, outs, rank, tuple(v["order"])) * tokens
+        want = 2 * (n_in * n_out * tokens + weight) if joined else chain
+        assert plan.launch_flops(index, tokens) == want, v["name"]
+        assert v["flops"] == chain
+    assert kinds == {False, True}
+    assert plan.launch_flops(-1, tokens) == plan.launch_flops(plan.select(tokens), tokens)
+    assert plan.launch_flops(plan.variant_count - 1, 0) == 0
+    with pytest.raises(_lib.TrkError):
+        plan.launch_flops(plan.variant_count, 1)
