@@ -197,7 +197,7 @@ int trk_forward_epilogue(const trk_plan *plan, int variant, const void *packed, 
  * packed_up their packed cores. Each workgroup computes its tile of G x, keeps it in fp32
  * registers, computes the same tile of U x and stores silu(G x) * (U x), rounded once to the
  * dtype; nothing is allocated and no intermediate reaches memory. The variant is gate's
- * selection for `tokens`. TRK_ERR_UNSUPPORTED when that variant has no fused kernel (fused
+ * selection for `tokens` among those with a fused kernel. TRK_ERR_UNSUPPORTED when none has one (fused
  * kernels are compiled for the declared gate/up shapes: the Llama-3-8B up projection and the
  * Qwen3.8-27B mlp_gate_up); a caller then runs the two projections with
  * trk_forward_epilogue (TRK_EPI_F32, then TRK_EPI_SILU_MUL). Replaces the reference's

@@ -15,8 +15,9 @@ const Entry kEntries[] = {
     TRK_ENTRY_PAIR(tile(kShape012, 1, 2, 28, 32, 4, 1, 2, 8, 32, 8, 1, 4), 17, 32)  // ring3_mfma_wide8x32w8p_s4<012,1,2,28,32,4,1,2>
     TRK_ENTRY_PAIR(tile(kShape012, 1, 2, 28, 32, 4, 2, 1, 8, 32, 8, 0, 4), 33, 64)  // ring3_mfma_wide8x32w8_s4<012,1,2,28,32,4,2,1>
     TRK_ENTRY_PAIR(tile(kShape012, 1, 8, 28, 32, 2, 2, 1, 8, 32, 8, 1), 65, 128)  // wide8x32w8_f8sc28k2n1_ic2_p
-    TRK_ENTRY_PAIR(tile(kShape012, 1, 8, 28, 32, 2, 2, 1, 8, 32, 8, 1), 193, 256)  // wide8x32w8_f8sc28k2n1_ic2_p
-    TRK_ENTRY_PAIR(tile(kShape012, 1, 8, 28, 32, 2, 2, 1, 8, 32, 8, 1), 321, 384)  // wide8x32w8_f8sc28k2n1_ic2_p
+    TRK_ENTRY_PAIR(tile(kShape012, 1, 8, 28, 32, 2, 2, 1, 8, 32, 8, 1), 193, 384)  // wide8x32w8_f8sc28k2n1_ic2_p
+    TRK_ENTRY_PAIR(tile(kShape012, 1, 8, 28, 32, 2, 2, 1, 8, 32, 8, 1), 1537, 1664)  // wide8x32w8_f8sc28k2n1_ic2_p
+    TRK_ENTRY_PAIR(tile(kShape012, 1, 8, 28, 32, 2, 2, 1, 8, 32, 8, 1), 2177, 2432)  // wide8x32w8_f8sc28k2n1_ic2_p
 };
 
 }  // namespace

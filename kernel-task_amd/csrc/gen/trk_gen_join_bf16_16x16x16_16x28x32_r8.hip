@@ -9,7 +9,7 @@ constexpr Shape kShape120{TRK_DTYPE_BF16, 1, 2, 0, 16, 16, 16, 16, 28, 32, 8};
 
 const Entry kEntries[] = {
     TRK_ENTRY_JOIN_PAIR(tile(kShape120, 96, 1, 8, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 129, 192)  // ring3_join_w8<120,96,1,8,16,1,2,1>
-    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 160, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 257, 320)  // ring3_join<120,160,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN(tile(kShape120, 160, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 257, 320)  // ring3_join<120,160,1,8,16,1,1,2>
     TRK_ENTRY_JOIN_PAIR(tile(kShape120, 112, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 385, 448)  // ring3_join_w8<120,112,2,8,16,1,1,1>
     TRK_ENTRY_JOIN_PAIR(tile(kShape120, 128, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 449, 512)  // ring3_join_w8<120,128,2,8,16,1,1,1>
     TRK_ENTRY_JOIN_PAIR(tile(kShape120, 160, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 513, 640)  // ring3_join_w8<120,160,2,8,16,1,1,1>
@@ -17,8 +17,11 @@ const Entry kEntries[] = {
     TRK_ENTRY_JOIN_PAIR(tile(kShape120, 128, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 769, 1024)  // ring3_join_w8<120,128,2,8,16,1,1,1>
     TRK_ENTRY_JOIN_PAIR(tile(kShape120, 144, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1025, 1280)  // ring3_join_w8<120,144,2,8,16,1,1,1>
     TRK_ENTRY_JOIN_PAIR(tile(kShape120, 176, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1281, 1536)  // ring3_join_w8<120,176,2,8,16,1,1,1>
-    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 160, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1537, 2048)  // ring3_join_w8<120,160,2,8,16,1,1,1>
-    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 176, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2049, 3072)  // ring3_join_w8<120,176,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 160, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1537, 1664)  // ring3_join_w8<120,160,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 160, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1665, 2048)  // ring3_join_w8<120,160,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 176, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2049, 2176)  // ring3_join_w8<120,176,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 176, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2305, 2432)  // ring3_join_w8<120,176,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN_PAIR(tile(kShape120, 176, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2433, 3072)  // ring3_join_w8<120,176,2,8,16,1,1,1>
     TRK_ENTRY_JOIN_PAIR(tile(kShape120, 192, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 3073, 1073741824)  // ring3_join_w8<120,192,2,8,16,1,1,1>
 };
 

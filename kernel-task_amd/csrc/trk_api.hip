@@ -52,27 +52,32 @@ void grid_of(const Plan &p, const Variant &v, int tokens, int grid[3]) {
 }
 
 // The variant of a call: later entries were registered for narrower token ranges (the joined-core
-// ones last) and win over earlier ones; gated ones count where the plan is admitted.
-int select_variant(const Plan &p, int tokens, bool admitted) {
+// ones last) and win over earlier ones; gated ones count where the plan is admitted. pair: among
+// those with a fused gate/up kernel, where there are any (a joined tile whose pair is slower than
+// that of the chain it lies over has none).
+int select_variant(const Plan &p, int tokens, bool admitted, bool pair = false) {
+    int alone = 0;
     for (int i = p.nvariants - 1; i > 0; --i) {
         const Variant &v = p.variants[i];
-        if (v.t_min > 0 && tokens >= v.t_min && tokens <= v.t_max && (admitted || !v.gated)) return i;
+        if (v.t_min <= 0 || tokens < v.t_min || tokens > v.t_max || (v.gated && !admitted)) continue;
+        if (!pair || v.launch_pair) return i;
+        if (!alone) alone = i;
     }
-    return 0;
+    return alone;
 }
 
 // The token range the default selection routes to variant i (0, 0: none): the range it holds, for
-// a gated variant of a plan that is not admitted none, and for the chain variants under admitted
-// gated ones without what those take at its ends.
+// a gated variant of a plan that is not admitted none, and for the chain variants under joined
+// ones without what those take at its ends.
 void routed_range(const Plan &p, int i, int *t_min, int *t_max) {
     int lo = p.variants[i].t_min, hi = p.variants[i].t_max;
     if (p.variants[i].gated && p.admitted <= 0) lo = hi = 0;
-    bool moved = p.admitted > 0 && !p.variants[i].gated && p.variants[i].kind == TRK_KERNEL_MFMA;
+    bool moved = p.variants[i].kind == TRK_KERNEL_MFMA && !p.chains[p.variants[i].chain].join;
     while (moved && lo > 0 && lo <= hi) {
         moved = false;
         for (int k = i + 1; k < p.nvariants; ++k) {
             const Variant &w = p.variants[k];
-            if (!w.gated || w.t_min <= 0) continue;
+            if (!p.chains[w.chain].join || w.t_min <= 0 || (w.gated && p.admitted <= 0)) continue;
             if (w.t_min <= lo && lo <= w.t_max) lo = w.t_max + 1, moved = true;
             if (w.t_min <= hi && hi <= w.t_max) hi = w.t_min - 1, moved = true;
         }
@@ -467,7 +472,7 @@ int trk_forward_swiglu(const trk_plan *gate, const void *packed_gate, const trk_
                          "trk_forward_swiglu: the gate and up plans differ in shape, dtype, rank "
                          "or packed layout");
     if (tokens == 0) return TRK_OK;
-    const Variant &v = g.variants[select_variant(g, tokens, g.admitted > 0 && u.admitted > 0)];
+    const Variant &v = g.variants[select_variant(g, tokens, g.admitted > 0 && u.admitted > 0, true)];
     const Chain &cg = g.chains[v.chain], &cu = u.chains[v.chain];
     if (cg.offF != cu.offF || cg.offS != cu.offS || cg.offL != cu.offL)
         return set_error(TRK_ERR_INVALID, "trk_forward_swiglu: the plans' packed layouts differ");

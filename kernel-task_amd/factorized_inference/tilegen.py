@@ -740,13 +740,13 @@ def neighbours(shape: ShapeDecl, order: tuple, t: Tile) -> dict[str, Tile]:
 
 
 def join_candidates(shape: ShapeDecl) -> dict[str, Tile]:
-    """The joined-core tiles worth timing (extended search). Few tokens: waves that split the
+    """The joined-core tiles worth timing (tilegen --joined). Few tokens: waves that split the
     features of 1-4 output pairs. Many: waves that share x over 4-16 pairs. Four waves of the
     largest tile a register file holds suit calls that fill the chip several times over; eight
     (one workgroup a CU) suit the calls of one or two rounds, where two waves a SIMD hide what
     one of them waits for."""
-    small, large = (16, 32, 48, 64, 96, 128), (64, 96, 128, 192, 256)
-    mid = (16, 32, 48, 64, 80, 96, 112, 128, 160, 192)
+    small, large = (16, 32, 48, 64, 80, 96, 112, 128), (64, 96, 128, 160, 192, 224, 240, 256)
+    mid = (16, 32, 48, 64, 80, 96, 112, 128, 144, 160, 176, 192)
     kinds = [(4, tt, fc, sc, 4) for tt in small for fc, sc in ((1, 1), (2, 1), (1, 2), (3, 1), (1, 4))]
     kinds += [(4, tt, fc, sc, 1) for tt in large for fc, sc in ((1, 4), (2, 4), (1, 8), (2, 8))]
     kinds += [(8, tt, fc, sc, kw) for tt in mid for kw, pairs in (
@@ -774,9 +774,6 @@ def search_candidates(shape: ShapeDecl, extended: bool = False) -> dict[str, tup
         tag = "" if order == first else "@" + order_tag(order)
         for name, t in candidates(shape, order, extended).items():
             out[name + tag] = (order, t)
-    if extended:
-        out |= {name + "@" + order_tag(JOIN_ORDER): (JOIN_ORDER, t)
-                for name, t in join_candidates(shape).items()}
     return out
 
 
@@ -793,23 +790,47 @@ def add_candidate(cands: dict, name: str, order: tuple, tile: Tile) -> str | Non
     return unique
 
 
+def left_of(lo: int, hi: int, taken: list[tuple[int, int]]) -> list[tuple[int, int]]:
+    """What the ranges `taken` leave of [lo, hi], as ranges in order."""
+    parts = [(lo, hi)]
+    for a, b in taken:
+        parts = [p for x, y in parts for p in ((x, min(y, a - 1)), (max(x, b + 1), y))
+                 if p[0] <= p[1]]
+    return parts
+
+
 def table(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = False,
-          extended: bool = False, admitted: bool = False) -> list[tuple[str, tuple, Tile, int, int]]:
+          extended: bool = False, admitted: bool = False,
+          joined: str = "") -> list[tuple[str, tuple, Tile, int, int]]:
     """[(name, order, tile, t_min, t_max)] for one shape: the tuned winners when the shape
     has measurements, else every candidate with the rule's ranges (0, 0: index only).
-    A tuned entry's "ranges" are its chain tiles, "joined" its joined-core tiles. In fp16 the
-    chains' ranges cover every token count and the joined tiles' lie over them, for plans whose
-    cores trk_plan_admit finds even; they are 0, 0 here unless `admitted` asks for them. Its "extra"
-    tiles are compiled index-only beside the winners (alternatives a caller may route token
-    counts to, such as the XCD-local tiles).
-    all_candidates=True ignores the measurements (the autotuner's input)."""
+    A tuned entry's "ranges" are its chain tiles, which cover every token count, "joined" its
+    joined-core tiles, which take theirs out of the chains' (a chain tile left without any is not
+    compiled); one whose fused pair is slower than the chain's ("pair" false) lies over the chain's
+    range, which trk_forward_swiglu keeps. In fp16 they lie over the chains' instead, for plans whose cores trk_plan_admit
+    finds even, and are 0, 0 here unless `admitted` asks for them. Its "extra" tiles are compiled
+    index-only beside the winners (alternatives a caller may route token counts to, such as the
+    XCD-local tiles).
+    all_candidates=True ignores the measurements (the autotuner's input for the chains). joined is
+    its input for the joined tiles: the chains with all of their ranges, and index-only the tiles
+    of join_candidates ("all") or the winners so far ("tuned")."""
     tuned = load_tuned() if tuned is None else tuned
     entry = None if all_candidates else tuned.get(shape.key)
     if entry:
-        rows = [(r["name"], tuple(r.get("order", entry["order"])), Tile(**r["tile"]),
-                 r["t_min"], r["t_max"]) for r in entry["ranges"] + entry.get("joined", [])]
-        if shape.dtype == "f16" and not admitted:
-            rows = [(n, o, t, 0, 0) if t.JN else (n, o, t, lo, hi) for n, o, t, lo, hi in rows]
+        chains, over, paired = (
+            [(r["name"], tuple(r.get("order", entry["order"])), Tile(**r["tile"]),
+              r["t_min"], r["t_max"]) for r in entry.get(key, []) if pair or r.get("pair", True)]
+            for key, pair in (("ranges", True), ("joined", True), ("joined", False)))
+        if joined:
+            tiles = {t: n for n, t in join_candidates(shape).items()} if joined == "all" else {}
+            tiles |= {t: n for n, _, t, _, _ in over}
+            rows = chains + [(n, JOIN_ORDER, t, 0, 0) for t, n in tiles.items()]
+        elif shape.dtype == "f16":
+            rows = chains + (over if admitted else [(n, o, t, 0, 0) for n, o, t, _, _ in over])
+        else:
+            taken = [(lo, hi) for *_, lo, hi in paired]
+            rows = [(n, o, t, *part) for n, o, t, lo, hi in chains
+                    for part in left_of(lo, hi, taken)] + over
         rows += [(r["name"], tuple(r.get("order", entry["order"])), Tile(**r["tile"]), 0, 0)
                  for r in entry.get("extra", [])]
         for name, order, t, _, _ in rows:
@@ -827,7 +848,7 @@ def table(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = Fa
         # stage 2 with the tail waves' issue priority (TP) and, for the register-resident
         # winners of 5 tokens or more, their neighbours (a local refinement)
         entry = tuned[shape.key]
-        for r in entry["ranges"] + entry.get("joined", []) + entry.get("extra", []):
+        for r in entry["ranges"] + entry.get("extra", []):
             order = tuple(r.get("order", entry["order"]))
             if order not in ORDERS:
                 continue
@@ -838,7 +859,7 @@ def table(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = Fa
             base, _, tag = name.partition("@")
             tag = "@" + tag if tag else ""
             found = [(name, tile)]
-            if extended and not tile.JN:
+            if extended:
                 found += [(base + suffix + tag, v)
                           for suffix, v in s1_variants(shape, order, tile).items()]
                 late = replace(tile, SL=1)
@@ -860,11 +881,11 @@ def _fn_name(shape: ShapeDecl, join: bool = False) -> str:
 
 
 def emit(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = False,
-         extended: bool = False, join: bool = False) -> str:
+         extended: bool = False, join: bool = False, joined: str = "") -> str:
     """One translation unit: the shape's chain tiles, or (join) its joined-core tiles, which
     build_ext compiles with other flags."""
     tuned = load_tuned() if tuned is None else tuned
-    rows = [r for r in table(shape, tuned, all_candidates, extended, admitted=True)
+    rows = [r for r in table(shape, tuned, all_candidates, extended, True, joined)
             if bool(r[2].JN) == join]
     orders = sorted({r[1] for r in rows}, key=lambda od: (od != choose_order(shape), od))
     i, o = shape.ins, shape.outs
@@ -888,8 +909,10 @@ def emit(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = Fal
                      f"{od[1]}, {od[2]}, {i[0]}, {i[1]}, {i[2]}, {o[0]}, {o[1]}, {o[2]}, "
                      f"{shape.rank}}};")
     lines += ["", "const Entry kEntries[] = {"]
+    alone = {r["t_min"] for r in tuned.get(shape.key, {}).get("joined", []) if not r.get("pair", True)}
     for name, od, t, lo, hi in rows:
-        macro = "TRK_ENTRY" + ("_JOIN" if t.JN else "") + ("_PAIR" if shape.swiglu else "")
+        pair = shape.swiglu and not (t.JN and lo in alone)
+        macro = "TRK_ENTRY" + ("_JOIN" if t.JN else "") + ("_PAIR" if pair else "")
         lines.append(f"    {macro}(tile(kShape{order_tag(od)}, {t.args()}), {lo}, {hi})  // {name}")
     lines += [
         "};",
@@ -944,28 +967,28 @@ def emit_index(shapes: list[ShapeDecl], joined: list[ShapeDecl] = []) -> str:
 
 
 def write_all(shapes: list[ShapeDecl] = DECLARED, out_dir: Path = GEN_DIR,
-              all_candidates: bool = False, extended: bool = False) -> list[Path]:
+              all_candidates: bool = False, extended: bool = False, joined: str = "") -> list[Path]:
     """Write one translation unit per shape plus the index; stale generated units are
     removed. Returns the written sources. all_candidates=True compiles every candidate with
-    rule ranges (for the autotuner) instead of the tuned winners."""
+    rule ranges (for the autotuner) instead of the tuned winners; joined as in table()."""
     out_dir.mkdir(parents=True, exist_ok=True)
     tuned = load_tuned()
-    written, joined = [], []
+    written, with_join = [], []
     for s in shapes:
         p = out_dir / f"trk_gen_{s.key}.hip"
-        text = emit(s, tuned, all_candidates, extended)
+        text = emit(s, tuned, all_candidates, extended, joined=joined)
         if not p.exists() or p.read_text() != text:
             p.write_text(text)
         written.append(p)
-        if any(r[2].JN for r in table(s, tuned, all_candidates, extended)):
-            joined.append(s)
+        if any(r[2].JN for r in table(s, tuned, all_candidates, extended, joined=joined)):
+            with_join.append(s)
             p = out_dir / f"trk_gen_join_{s.key}.hip"
-            text = emit(s, tuned, all_candidates, extended, join=True)
+            text = emit(s, tuned, all_candidates, extended, join=True, joined=joined)
             if not p.exists() or p.read_text() != text:
                 p.write_text(text)
             written.append(p)
     index = out_dir / "trk_gen_index.hip"
-    text = emit_index(shapes, joined)
+    text = emit_index(shapes, with_join)
     if not index.exists() or index.read_text() != text:
         index.write_text(text)
     written.append(index)
@@ -994,5 +1017,7 @@ if __name__ == "__main__":
     import sys
 
     for path in write_all(all_candidates="--all" in sys.argv[1:],
-                          extended="--extended" in sys.argv[1:]):
+                          extended="--extended" in sys.argv[1:],
+                          joined="all" if "--joined" in sys.argv[1:] else
+                          "tuned" if "--joined-tuned" in sys.argv[1:] else ""):
         print(path)

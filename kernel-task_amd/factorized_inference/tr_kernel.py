@@ -294,8 +294,8 @@ def forward_swiglu(gate: PreparedTRKernel, up: PreparedTRKernel, x: torch.Tensor
     """silu(gate(x)) * up(x), the gate and up projections of a SwiGLU block, in the cores'
     dtype from one launch (trk_forward_swiglu): each workgroup computes its tile of gate(x),
     keeps it in fp32 registers, computes the same tile of up(x) and stores the product,
-    rounded once. Where the plan's selected variant has no fused kernel (shapes other than
-    the declared gate/up ones), the same result comes from two launches:
+    rounded once. Where none of the plan's variants for the count has a fused kernel (shapes other
+    than the declared gate/up ones), the same result comes from two launches:
     up.forward_silu_mul(x, gate.accumulate(x)). Reference: the accumulate / accumulate /
     consume_silu_mul chain of csrc/v3g/bind.cu:84-136, which takes three launches."""
     if not isinstance(gate, PreparedTRKernel) or not isinstance(up, PreparedTRKernel):

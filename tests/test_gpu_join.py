@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from factorized_inference import TRSpec, _lib, make_cores, prepare_optimized
+from factorized_inference import TRSpec, _lib, make_cores, prepare_optimized, tilegen
 from factorized_inference.tr_kernel import current_stream_handle, forward_swiglu
 import join_model as jm
 from gpu_util import check_result, oracle_y
@@ -150,6 +150,68 @@ def test_swiglu_pair_of_joined_tiles():
         x = torch.randn(t, spec.in_features, device="cuda", dtype=dtype,
                         generator=torch.Generator(device="cuda").manual_seed(t))
         assert torch.equal(forward_swiglu(gate, up, x), up.forward_silu_mul(x, gate.accumulate(x)))
+
+
+@pytest.mark.parametrize("shape,rank", [("llama_up", 8), ("gate_up", 8), ("gate_up", 16)])
+def test_swiglu_pair_of_every_joined_tile(shape, rank):
+    # at a token tile's edge and just past it: the fused kernel against the two launches of the same
+    # tile, and the oracle on sampled rows. Tiles of 3 output digits overhang oQ = 34, and at
+    # 48 tokens over 4 waves a share of the tiles is uneven.
+    ins, outs = {"llama_up": ((16, 16, 16), (16, 28, 32)), "gate_up": SHAPES["gate_up_r8"][:2]}[shape]
+    spec, dtype = TRSpec(ins, outs, rank), torch.bfloat16
+    cores = [make_cores(spec, device="cuda", dtype=dtype, seed=s) for s in (13, 14)]
+    gate, up = (prepare_optimized(c, spec) for c in cores)
+    lib, stream = _lib.load(), current_stream_handle(gate.device_index)
+    x_all = torch.randn(257, spec.in_features, device="cuda", dtype=dtype,
+                        generator=torch.Generator(device="cuda").manual_seed(15))
+    tiles: dict = {}
+    for i, v in enumerate(gate.variants()):
+        if "join" in v["name"]:
+            tiles.setdefault(v["name"], (v["tile"][0], []))[1].append(i)
+    rows = sorted({r for tt, _ in tiles.values() for r in (0, tt - 1, tt)})
+    g, u = (dict(zip(rows, oracle_y(x_all[rows], c, spec))) for c in cores)
+    decl = next(d for d in tilegen.DECLARED if d.swiglu and (d.ins, d.outs, d.rank) == (ins, outs, rank))
+    paired = {r["name"] for r in tilegen.load_tuned()[decl.key]["joined"] if r.get("pair", True)}
+    assert len(paired) >= 7 and paired <= set(tiles)
+    for name, (tt, indices) in tiles.items():
+        for t in (tt, tt + 1):
+            print("case:", shape, rank, name, t, flush=True)
+            x, y = x_all[:t].clone(), torch.empty(t, spec.out_features, device="cuda", dtype=dtype)
+            fused = 0
+            for i in indices:  # one per token range; those whose pair the chains serve have no kernel
+                gate.plan.set_variant(1, 1 << 30, i)
+                status = lib.trk_forward_swiglu(
+                    gate.plan.handle, gate.packed.data_ptr(), up.plan.handle, up.packed.data_ptr(),
+                    x.data_ptr(), y.data_ptr(), t, stream)
+                assert status in (_lib.OK, _lib.ERR_UNSUPPORTED)
+                fused += status == _lib.OK
+            assert bool(fused) == (name in paired), name
+            if not fused:
+                continue
+            two = up.run_variant(x, indices[0], _lib.EPI_SILU_MUL,
+                                 gate.run_variant(x, indices[0], _lib.EPI_F32))
+            assert torch.equal(y, two), (name, t)
+            at = sorted({0, tt - 1, t - 1})
+            gv, uv = (np.stack([d[r] for r in at]) for d in (g, u))
+            want = gv / (1 + np.exp(-gv)) * uv
+            # each factor is REL off; silu's slope is at most 1.1 and |g| about twice |silu(g)|
+            err = np.linalg.norm(y[at].double().cpu().numpy() - want)
+            assert err <= 3 * REL[dtype] * np.linalg.norm(want), (name, t)
+
+
+def test_swiglu_pair_keeps_the_chain_where_it_is_faster():
+    # 4096 -> 14336 at 300 tokens: the plain call runs a joined tile, the fused pair the chain's
+    # (124.9 against 126.9 us), which is the one it ran before that tile took the range
+    spec, dtype = TRSpec((16, 16, 16), (16, 28, 32), 8), torch.bfloat16
+    gate, up = (prepare_optimized(make_cores(spec, device="cuda", dtype=dtype, seed=s), spec)
+                for s in (16, 17))
+    x = torch.randn(300, spec.in_features, device="cuda", dtype=dtype)
+    assert "join" in gate.selected(300)["name"]
+    chain = gate.selected(350)
+    assert "join" not in chain["name"]
+    index = gate.plan.select(350)
+    want = up.run_variant(x, index, _lib.EPI_SILU_MUL, gate.run_variant(x, index, _lib.EPI_F32))
+    assert torch.equal(forward_swiglu(gate, up, x), want)
 
 
 def test_captured_joined_launch_replays():

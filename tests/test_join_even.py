@@ -1,6 +1,6 @@
-"""CPU checks of where fp16 plans may use joined-core tiles: a model of both kernels' roundings over
+"""CPU checks of where plans use joined-core tiles. fp16: a model of both kernels' roundings over
 cores that are even and uneven in every way the rule looks at, and what a plan routes before and after
-trk_plan_admit. On the GPU: tests/test_gpu_join.py."""
+trk_plan_admit. SwiGLU shapes: the tiles that leave the fused pair to the chains. On the GPU: tests/test_gpu_join.py."""
 from __future__ import annotations
 
 import pytest
@@ -67,3 +67,21 @@ def test_admit_refuses_null_and_leaves_other_dtypes_alone():
     assert "join" in before[-1]
     assert lib.trk_plan_admit(plan.handle, 256, None) == _lib.OK  # not read
     assert before == [plan.describe(-1, t)["name"] for t in (1, 64, 512)]
+
+
+@pytest.mark.parametrize("shape", [s for s in tilegen.DECLARED if s.swiglu], ids=lambda s: s.key)
+def test_every_count_of_a_swiglu_shape_has_a_fused_pair(shape):
+    # a joined row without a pair kernel lies over a chain row, which has one
+    entry = tilegen.load_tuned()[shape.key]
+    rows = tilegen.table(shape)
+    alone = [r for r in entry["joined"] if not r.get("pair", True)]
+    for r in alone:
+        assert any(lo <= r["t_min"] and r["t_max"] <= hi for _, _, t, lo, hi in rows if not t.JN)
+    text = tilegen.emit(shape, join=True)
+    assert text.count("TRK_ENTRY_JOIN(") == len(alone)
+    assert text.count("TRK_ENTRY_JOIN_PAIR(") == len(entry["joined"]) - len(alone)
+    plan = _lib.Plan(shape.ins, shape.outs, shape.rank, _lib.DTYPE_BF16)
+    for r in entry["joined"]:
+        for t in (r["t_min"], r["t_max"]):
+            info = plan.describe(-1, t)
+            assert info["name"] == r["name"] and (info["t_min"], info["t_max"]) == (r["t_min"], r["t_max"])
