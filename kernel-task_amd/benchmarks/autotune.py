@@ -2,7 +2,7 @@
 declared shape over a grid of token counts and write the fastest per token range.
 
     python -m factorized_inference.tilegen --all   # compile every candidate (from kernel-task_amd/)
-    python -m factorized_inference.build_ext
+    python -m factorized_inference.build_ext --as-generated
     python kernel-task_amd/benchmarks/autotune.py --out OUT/tuned.json    # on an MI355X
         (the winners' table; the raw timings of every candidate go to --measurements, a file
         outside the source tree, and never into the tables)
@@ -30,6 +30,12 @@ as equal, and then the tile on the fewest XCDs wins (Tile.XL).
 Candidates span every chain order the generator searches (tilegen.search_orders); each
 range records its winner's order. Token counts measured: 1, 2, 4, 8, 16, 32, 64, 128, 256. The winner at T serves the range
 (previous measured T, T]; 256's winner serves everything above.
+
+The joined-core tiles take their ranges out of the chains' in a pass of their own, once those are
+tuned: `tilegen --joined` (every candidate) or `--joined-tuned` (the winners so far, to measure
+their ranges again), a build as above, then `--joined`. It times them beside the chain of each
+count, eagerly and on rotating inputs, at both ends of the ranges JOIN_EDGES bounds (--held: each
+tuned tile at its own counts only); see joined_rows for the rule, tune_joined for what is timed.
 """
 from __future__ import annotations
 
@@ -49,6 +55,7 @@ sys.path.insert(0, str(PACKAGE_ROOT))
 import torch  # noqa: E402
 
 from factorized_inference import TRSpec, make_cores, prepare_optimized, tilegen  # noqa: E402
+from factorized_inference.tr_kernel import forward_swiglu  # noqa: E402
 
 GRID = (1, 2, 4, 8, 16, 32, 64, 128, 256)
 
@@ -120,7 +127,8 @@ def tune_shape(shape: tilegen.ShapeDecl, budget_s: float,
     spec = TRSpec(shape.ins, shape.outs, shape.rank)
     cores = make_cores(spec, device="cuda", dtype=dtype, seed=0, init="uniform")
     run = prepare_optimized(cores, spec)
-    variants = [(i, v) for i, v in enumerate(run.variants()) if v["kind"] == "mfma"]
+    variants = [(i, v) for i, v in enumerate(run.variants())
+                if v["kind"] == "mfma" and "join" not in v["name"]]
     names, tiles = {}, {}
     cands = tilegen.search_candidates(shape, extended=True)
     for i, v in variants:
@@ -189,11 +197,153 @@ def tune_shape(shape: tilegen.ShapeDecl, budget_s: float,
     for r in ranges:
         r["order"] = list(tiles[r["name"]][0])
         r["tile"] = asdict(tiles[r["name"]][1])
-    joined = [r for r in ranges if r["tile"]["JN"]]
-    return ({"order": list(order), "device": torch.cuda.get_device_name(0),
-             "ranges": [r for r in ranges if not r["tile"]["JN"]],
-             **({"joined": joined} if joined else {})},
+    return ({"order": list(order), "device": torch.cuda.get_device_name(0), "ranges": ranges},
             {str(T): row for T, row in measured.items()})
+
+
+# Ends of the ranges joined tiles are chosen for: their cost steps at multiples of their token
+# tiles, which are multiples of 16, and the steps that matter grow with the count.
+JOIN_EDGES = [*range(16, 512, 16), *range(512, 1024, 32), *range(1024, 2048, 64),
+              *range(2048, 4097, 128)]
+JOIN_GAIN, JOIN_STAY = 0.03, 0.01
+
+
+def able_tiles(calls: dict[str, dict[str, float]]) -> list[str]:
+    """The joined tiles of one token count's timings (us[call][tile], see joined_rows) that are at
+    least JOIN_GAIN faster than the chain and, where the epilogues were timed too, not slower
+    there on average."""
+    plain = calls["plain"]
+    epilogues = [c for call, c in calls.items() if call not in ("plain", "pair")]
+    return [n for n, v in plain.items() if n != "chain" and v * (1 + JOIN_GAIN) <= plain["chain"]
+            and sum(c.get(n, c["chain"]) / c["chain"] for c in epilogues) <= len(epilogues)]
+
+
+def joined_rows(edges: list[int], us: dict[int, dict[str, dict[str, float]]]) -> list[dict]:
+    """Joined tiles' token ranges from us[T][call][tile], microseconds per call at both ends of
+    every range (edges[k - 1], edges[k]]; the tile "chain" is the chain that serves T without
+    them, the call "plain" is timed for every tile, others at lower ends alone. A tile may take a
+    range it is able to at both ends (able_tiles). The least sum over the ends wins, but the
+    winner of the range below stays within JOIN_STAY of it. Where the fused pair is slower than the
+    chain's ("pair" false), trk_forward_swiglu keeps the chain's. The last range has no end."""
+    rows: list[dict] = []
+    for k, hi in enumerate(edges):
+        lo = edges[k - 1] + 1 if k else 1
+        if lo not in us or hi not in us:
+            continue
+        high = able_tiles(us[hi])
+        able = {n: us[lo]["plain"][n] + us[hi]["plain"][n] for n in able_tiles(us[lo]) if n in high}
+        if not able:
+            continue
+        best = min(able, key=able.get)
+        if rows and rows[-1]["t_max"] == lo - 1:
+            last = rows[-1]["name"]
+            if able.get(last, float("inf")) <= able[best] * (1 + JOIN_STAY):
+                best = last
+        row = {"name": best, "t_min": lo, "t_max": hi}
+        pair = us[lo].get("pair", {})
+        if pair.get(best, 0.0) > pair.get("chain", 0.0):
+            row["pair"] = False
+        if rows and {**rows[-1], "t_min": lo, "t_max": hi} == row and rows[-1]["t_max"] == lo - 1:
+            rows[-1]["t_max"] = hi
+        else:
+            rows.append(row)
+    if rows and rows[-1]["t_max"] == edges[-1]:
+        rows[-1]["t_max"] = 1 << 30
+    return rows
+
+
+def rotating_us(fns: list, block_us: float = 6e3) -> float:
+    """Time per call of back-to-back calls that take `fns` in turn, median of three blocks after
+    one that warms up (what is timed first after an idle spell reads 5-10 % slow)."""
+    fns[0]()
+    torch.cuda.synchronize()
+    t0 = time.perf_counter()
+    fns[0]()
+    torch.cuda.synchronize()
+    calls = max(3, min(600, int(block_us / max((time.perf_counter() - t0) * 1e6, 4.0))))
+    out = []
+    for _ in range(4):
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        for k in range(calls):
+            fns[k % len(fns)]()
+        torch.cuda.synchronize()
+        out.append((time.perf_counter() - t0) * 1e6 / calls)
+    return statistics.median(out[1:])
+
+
+def tune_joined(shape: tilegen.ShapeDecl, held: list[dict] | None = None) -> tuple[list[dict], dict]:
+    """The joined tiles' rows of a plan that holds them index-only beside the chains' ranges, and
+    the timings behind them. held: rows whose tiles keep their token counts where they are able
+    to; None searches all the plan's joined tiles. Tiles are timed in turn with the chain, there
+    and back, the smaller time counting. Within a range whose lower end is still the chain's, the
+    first count the joined tile takes is found by bisection. At the lower ends the fp32 store,
+    the gate product (fp32 gate) and the SwiGLU shapes' fused pair are timed as well."""
+    dtype = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[shape.dtype]
+    tol = 1e-4 if dtype is torch.float32 else 0.02
+    spec = TRSpec(shape.ins, shape.outs, shape.rank)
+    runs = [prepare_optimized(make_cores(spec, device="cuda", dtype=dtype, seed=s), spec)
+            for s in range(2 if shape.swiglu else 1)]
+    run = runs[0]
+    joined = {v["name"]: i for i, v in enumerate(run.variants()) if "join" in v["name"]}
+    gen = torch.Generator(device="cuda").manual_seed(shape.rank)
+    xs = [torch.randn(JOIN_EDGES[-1], spec.in_features, device="cuda", generator=gen).to(dtype)
+          for _ in range(3)]
+    gate = torch.randn(JOIN_EDGES[-1], spec.out_features, device="cuda", generator=gen)
+    chains = [run.plan.select(T) for T in range(JOIN_EDGES[-1] + 1)]  # before any routing below
+    calls = {"plain": lambda x: run(x), "f32": lambda x: run.accumulate(x),
+             "silu_mul": lambda x: run.forward_silu_mul(x, gate[:len(x)])}
+    if shape.swiglu:
+        calls["pair"] = lambda x: forward_swiglu(run, runs[1], x)
+    us: dict[int, dict[str, dict[str, float]]] = {}
+
+    def timed(T: int, call: str, names: list[str]) -> dict[str, float]:
+        out: dict[str, float] = {}
+        x = [v[:T] for v in xs]
+        for n in [*names, *reversed(names)]:
+            run.plan.set_variant(1, 1 << 30, chains[T] if n == "chain" else joined[n])
+            v = rotating_us([lambda x=x: calls[call](x) for x in x])
+            out[n] = min(v, out.get(n, v))
+        return out
+
+    def measure(T: int, lower: bool) -> list[str]:
+        names = [n for n in joined if held is None or any(
+            r["name"] == n and r["t_min"] <= T <= r["t_max"] for r in held)]
+        ref = run.run_variant(xs[0][:T], chains[T]).float() if names else None
+        for n in list(names):
+            y = run.run_variant(xs[0][:T], joined[n]).float()
+            if not (y - ref).abs().max() <= tol * ref.abs().max() + tol:
+                print(f"  {shape.key} T={T} {n}: disagrees, skipped", flush=True)
+                names.remove(n)
+        us[T] = {"plain": timed(T, "plain", ["chain", *names]) if names else {"chain": 0.0}}
+        able = able_tiles(us[T])
+        if lower and able:
+            best = min(us[T]["plain"].values())
+            close = [n for n in able if us[T]["plain"][n] <= 1.05 * best]
+            for call in list(calls)[1:]:
+                us[T][call] = timed(T, call, ["chain", *close])
+        print(f"{shape.key} T={T}: " + "  ".join(f"{n} {v:.2f}" for n, v in sorted(
+            us[T]["plain"].items(), key=lambda kv: kv[1])[:4]), flush=True)
+        return able_tiles(us[T])
+
+    edges, lo = [], 1
+    for hi in JOIN_EDGES:
+        at_hi = measure(hi, False)
+        if at_hi and not set(measure(lo, True)) & set(at_hi):
+            below, above = lo, hi  # the chain's, a joined tile's
+            while above - below > 1:
+                mid = (below + above) // 2
+                if set(measure(mid, True)) & set(at_hi):
+                    above = mid
+                else:
+                    below = mid
+            if above < hi:
+                edges.append(above - 1)
+        edges.append(hi)
+        lo = hi + 1
+    rows = [{**r, "order": list(tilegen.JOIN_ORDER),
+             "tile": asdict(tilegen.parse_variant_name(r["name"])[1])} for r in joined_rows(edges, us)]
+    return rows, {"edges": edges, "us": us}
 
 
 def main() -> int:
@@ -206,6 +356,12 @@ def main() -> int:
                          "every tile). Graph replays keep the L2 warm across kernels where eager "
                          "launches do not, which ranked tiles differently on MI355X: one that "
                          "shares fewer core slices per XCD won graph replays and lost eager calls")
+    ap.add_argument("--joined", action="store_true",
+                    help="choose the joined-core tiles' ranges (a build of tilegen --joined or "
+                         "--joined-tuned) instead of the chains'")
+    ap.add_argument("--held", action="store_true",
+                    help="with --joined: keep the tuned rows' tiles and measure only where they "
+                         "are faster than the chains")
     ap.add_argument("--measurements", type=Path, default=Path("gpurun_out/autotune_us.json"),
                     help="where the raw per-candidate timings go (not part of the tables)")
     args = ap.parse_args()
@@ -228,10 +384,14 @@ def main() -> int:
             if wanted and shape.key not in wanted:
                 continue
             prev = result.get(shape.key) or tilegen.load_tuned().get(shape.key) or {}
-            result[shape.key], raw[shape.key] = tune_shape(shape, args.seconds_per_shape,
-                                                           args.eager_from_us)
-            if prev.get("extra"):  # index-only alternatives outlive a retune
-                result[shape.key]["extra"] = prev["extra"]
+            if args.joined:
+                rows, raw[shape.key] = tune_joined(shape, prev.get("joined") if args.held else None)
+                result[shape.key] = {**prev, "joined": rows}
+            else:
+                result[shape.key], raw[shape.key] = tune_shape(shape, args.seconds_per_shape,
+                                                               args.eager_from_us)
+                # index-only alternatives and the joined tiles' ranges outlive a retune
+                result[shape.key] |= {k: prev[k] for k in ("extra", "joined") if prev.get(k)}
             for path, data in ((args.out, result), (args.measurements, raw)):
                 path.parent.mkdir(parents=True, exist_ok=True)
                 path.write_text(json.dumps(data, indent=1, sort_keys=True) + "\n")

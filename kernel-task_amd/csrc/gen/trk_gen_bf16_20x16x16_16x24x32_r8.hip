@@ -13,7 +13,11 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape012, 1, 1, 24, 32, 8, 2, 1, 8, 32, 8), 5, 8)  // wide8x32w8_t1k2n1_ic8
     TRK_ENTRY(tile(kShape012, 1, 1, 24, 32, 8, 1, 2, 8, 32, 8), 9, 16)  // wide8x32w8_t1k1n2_ic8
     TRK_ENTRY(tile(kShape012, 1, 2, 24, 32, 8, 1, 2, 8, 32, 8), 17, 32)  // wide8x32w8_f2k1n2_ic8
-    TRK_ENTRY(tile(kShape012, 1, 2, 24, 32, 4, 1, 2, 4, 32, 4), 33, 448)  // wide4x32_f2k1n2_ic4
+    TRK_ENTRY(tile(kShape012, 1, 2, 24, 32, 4, 1, 2, 4, 32, 4), 33, 476)  // wide4x32_f2k1n2_ic4
+    TRK_ENTRY(tile(kShape012, 1, 2, 24, 32, 4, 1, 2, 4, 32, 4), 513, 536)  // wide4x32_f2k1n2_ic4
+    TRK_ENTRY(tile(kShape012, 1, 2, 24, 32, 4, 1, 2, 4, 32, 4), 769, 928)  // wide4x32_f2k1n2_ic4
+    TRK_ENTRY(tile(kShape012, 1, 2, 24, 32, 4, 1, 2, 4, 32, 4), 1537, 1568)  // wide4x32_f2k1n2_ic4
+    TRK_ENTRY(tile(kShape012, 1, 2, 24, 32, 4, 1, 2, 4, 32, 4), 2049, 2179)  // wide4x32_f2k1n2_ic4
 };
 
 }  // namespace

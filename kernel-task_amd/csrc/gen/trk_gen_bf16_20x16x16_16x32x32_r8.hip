@@ -13,8 +13,9 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape012, 1, 1, 32, 32, 8, 1, 2, 8, 32, 8), 3, 8)  // wide8x32w8_t1k1n2_ic8
     TRK_ENTRY(tile(kShape012, 1, 1, 32, 32, 8, 2, 1, 8, 32, 8, 1), 9, 16)  // wide8x32w8_t1k2n1_ic8_p
     TRK_ENTRY(tile(kShape012, 1, 2, 32, 32, 8, 1, 2, 8, 32, 8), 17, 32)  // wide8x32w8_f2k1n2_ic8
-    TRK_ENTRY(tile(kShape012, 1, 2, 32, 32, 4, 1, 2, 4, 32, 4), 33, 1280)  // wide4x32_f2k1n2_ic4
-    TRK_ENTRY(tile(kShape012, 1, 2, 32, 32, 4, 1, 2, 4, 32, 4), 1537, 2048)  // wide4x32_f2k1n2_ic4
+    TRK_ENTRY(tile(kShape012, 1, 2, 32, 32, 4, 1, 2, 4, 32, 4), 33, 1472)  // wide4x32_f2k1n2_ic4
+    TRK_ENTRY(tile(kShape012, 1, 2, 32, 32, 4, 1, 2, 4, 32, 4), 1537, 2194)  // wide4x32_f2k1n2_ic4
+    TRK_ENTRY(tile(kShape012, 1, 2, 32, 32, 4, 1, 2, 4, 32, 4), 2305, 2822)  // wide4x32_f2k1n2_ic4
     TRK_ENTRY(tile(kShape012, 1, 2, 32, 32, 4, 1, 2, 4, 32, 4), 3073, 1073741824)  // wide4x32_f2k1n2_ic4
 };
 

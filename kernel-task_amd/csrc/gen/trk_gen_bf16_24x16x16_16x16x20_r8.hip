@@ -16,7 +16,8 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape012, 1, 2, 16, 20, 4, 1, 2, 4, 32, 8, 2), 17, 32)  // wide4x32w8_f2k1n2_ic4_p2
     TRK_ENTRY(tile(kShape012, 1, 2, 16, 20, 4, 1, 2, 4, 32, 8), 33, 128)  // wide4x32w8_f2k1n2_ic4
     TRK_ENTRY(tile(kShape012, 1, 2, 16, 20, 4, 1, 2, 8, 32, 8), 129, 160)  // wide8x32w8_f2k1n2_ic4
-    TRK_ENTRY(tile(kShape012, 1, 2, 16, 20, 4, 1, 2, 8, 32, 8), 193, 256)  // wide8x32w8_f2k1n2_ic4
+    TRK_ENTRY(tile(kShape012, 1, 2, 16, 20, 4, 1, 2, 8, 32, 8), 193, 288)  // wide8x32w8_f2k1n2_ic4
+    TRK_ENTRY(tile(kShape012, 1, 2, 16, 20, 4, 1, 2, 8, 32, 8), 385, 409)  // wide8x32w8_f2k1n2_ic4
 };
 
 }  // namespace

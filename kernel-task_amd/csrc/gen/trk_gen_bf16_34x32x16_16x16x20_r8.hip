@@ -12,7 +12,7 @@ const Entry kEntries[] = {
     TRK_ENTRY(tile(kShape012, 1, 1, 4, 10, 8, 8, 1, 0, 16, 8), 2, 2)  // t1_l10_s4_w8_k8
     TRK_ENTRY(tile(kShape012, 1, 1, 16, 20, 4, 2, 1, 8, 32, 8, 1), 3, 8)  // wide8x32w8_t1k2n1_ic4_p
     TRK_ENTRY(tile(kShape012, 1, 1, 16, 20, 4, 1, 2, 8, 32, 8), 9, 16)  // wide8x32w8_t1k1n2_ic4
-    TRK_ENTRY(tile(kShape012, 1, 2, 16, 20, 4, 1, 2, 8, 32, 8, 1), 17, 256)  // wide8x32w8_f2k1n2_ic4_p
+    TRK_ENTRY(tile(kShape012, 1, 2, 16, 20, 4, 1, 2, 8, 32, 8, 1), 17, 288)  // wide8x32w8_f2k1n2_ic4_p
 };
 
 }  // namespace

@@ -8,13 +8,14 @@ namespace {
 constexpr Shape kShape120{TRK_DTYPE_BF16, 1, 2, 0, 20, 16, 16, 16, 24, 32, 8};
 
 const Entry kEntries[] = {
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 449, 640)  // ring3_join_w8<120,128,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 477, 512)  // ring3_join_w8<120,128,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 537, 640)  // ring3_join_w8<120,128,2,8,16,1,1,1>
     TRK_ENTRY_JOIN(tile(kShape120, 160, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 641, 768)  // ring3_join_w8<120,160,2,8,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 769, 1024)  // ring3_join<120,128,1,8,16,1,1,2>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 16, 1, 1, 2, 0, 16, 4, 0, 0, 0, 0, 0, 0, 1), 929, 1024)  // ring3_join<120,128,1,8,16,1,1,2>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1025, 1280)  // ring3_join_w8<120,128,2,8,16,1,1,1>
     TRK_ENTRY_JOIN(tile(kShape120, 160, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1281, 1536)  // ring3_join_w8<120,160,2,8,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1537, 2048)  // ring3_join_w8<120,128,2,8,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2049, 3072)  // ring3_join_w8<120,192,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1569, 2048)  // ring3_join_w8<120,128,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2180, 3072)  // ring3_join_w8<120,192,2,8,16,1,1,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 3073, 1073741824)  // ring3_join_w8<120,128,2,8,16,1,1,1>
 };
 

@@ -8,8 +8,9 @@ namespace {
 constexpr Shape kShape120{TRK_DTYPE_BF16, 1, 2, 0, 20, 16, 16, 16, 32, 32, 8};
 
 const Entry kEntries[] = {
-    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1281, 1536)  // ring3_join_w8<120,192,2,8,16,1,1,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2049, 3072)  // ring3_join_w8<120,192,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1473, 1536)  // ring3_join_w8<120,192,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2195, 2304)  // ring3_join_w8<120,192,2,8,16,1,1,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 192, 2, 8, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 2823, 3072)  // ring3_join_w8<120,192,2,8,16,1,1,1>
 };
 
 }  // namespace

@@ -9,8 +9,8 @@ constexpr Shape kShape120{TRK_DTYPE_BF16, 1, 2, 0, 24, 16, 16, 16, 16, 20, 8};
 
 const Entry kEntries[] = {
     TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 4, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 161, 192)  // ring3_join_w8<120,64,1,4,16,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 257, 384)  // ring3_join_w8<120,128,1,4,16,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 96, 2, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 385, 512)  // ring3_join_w8<120,96,2,4,16,1,2,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 289, 384)  // ring3_join_w8<120,128,1,4,16,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 96, 2, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 410, 512)  // ring3_join_w8<120,96,2,4,16,1,2,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 513, 768)  // ring3_join_w8<120,128,2,4,16,1,2,1>
     TRK_ENTRY_JOIN(tile(kShape120, 96, 4, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 769, 1024)  // ring3_join_w8<120,96,4,4,16,1,1,1>
     TRK_ENTRY_JOIN(tile(kShape120, 112, 4, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1025, 1280)  // ring3_join_w8<120,112,4,4,16,1,1,1>

@@ -8,7 +8,7 @@ namespace {
 constexpr Shape kShape120{TRK_DTYPE_BF16, 1, 2, 0, 34, 32, 16, 16, 16, 20, 8};
 
 const Entry kEntries[] = {
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 257, 384)  // ring3_join_w8<120,128,1,4,16,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 16, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 289, 384)  // ring3_join_w8<120,128,1,4,16,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 96, 2, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 385, 448)  // ring3_join_w8<120,96,2,4,16,1,2,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 2, 4, 16, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 449, 768)  // ring3_join_w8<120,128,2,4,16,1,2,1>
     TRK_ENTRY_JOIN(tile(kShape120, 96, 4, 4, 16, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 769, 1024)  // ring3_join_w8<120,96,4,4,16,1,1,1>

@@ -8,10 +8,10 @@ namespace {
 constexpr Shape kShape120{TRK_DTYPE_F16, 1, 2, 0, 8, 12, 20, 12, 10, 24, 8};
 
 const Entry kEntries[] = {
-    TRK_ENTRY_JOIN(tile(kShape120, 48, 1, 2, 12, 1, 8, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 81, 96)  // ring3_join_w8<120,48,1,2,12,1,8,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 48, 1, 2, 12, 1, 8, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 86, 96)  // ring3_join_w8<120,48,1,2,12,1,8,1>
     TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 2, 12, 1, 8, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 97, 128)  // ring3_join_w8<120,64,1,2,12,1,8,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 4, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 161, 256)  // ring3_join_w8<120,64,1,4,12,1,4,1>
-    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 257, 512)  // ring3_join_w8<120,128,1,4,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 64, 1, 4, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 171, 256)  // ring3_join_w8<120,64,1,4,12,1,4,1>
+    TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 4, 12, 1, 4, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 262, 512)  // ring3_join_w8<120,128,1,4,12,1,4,1>
     TRK_ENTRY_JOIN(tile(kShape120, 96, 2, 4, 12, 1, 2, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 513, 768)  // ring3_join_w8<120,96,2,4,12,1,2,1>
     TRK_ENTRY_JOIN(tile(kShape120, 128, 1, 8, 12, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 769, 1024)  // ring3_join_w8<120,128,1,8,12,1,1,1>
     TRK_ENTRY_JOIN(tile(kShape120, 96, 2, 8, 12, 1, 1, 1, 0, 16, 8, 0, 0, 0, 0, 0, 0, 1), 1025, 1536)  // ring3_join_w8<120,96,2,8,12,1,1,1>

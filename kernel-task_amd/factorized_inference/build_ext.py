@@ -52,12 +52,14 @@ def file_flags(src: Path) -> list[str]:
     return HIPCC_FLAGS[:k - 1] + HIPCC_FLAGS[k + 1:]
 
 
-def sources() -> list[Path]:
+def sources(regenerate: bool = True) -> list[Path]:
     """Every HIP source: the hand-written ones and the generated variant tables (csrc/gen/,
-    rewritten from tilegen.py's declared shapes and tuned table first)."""
+    rewritten from tilegen.py's declared shapes and tuned table first; regenerate=False takes
+    them as they are, for a table of candidates that tilegen has written to be timed)."""
     from . import tilegen
 
-    tilegen.write_all()
+    if regenerate:
+        tilegen.write_all()
     return sorted(CSRC.glob("*.hip")) + sorted((CSRC / "gen").glob("*.hip"))
 
 
@@ -74,7 +76,8 @@ def _hipcc() -> str:
     return str(path) if path.exists() else "hipcc"
 
 
-def build(verbose: bool = False, jobs: int = 8, incremental: bool = False) -> Path:
+def build(verbose: bool = False, jobs: int = 8, incremental: bool = False,
+          regenerate: bool = True) -> Path:
     """Compile every source and link libtrk.so and the two bindings. incremental=True
     (development only) reuses objects newer than their source, the headers and this script."""
     OBJ_DIR.mkdir(exist_ok=True)
@@ -97,7 +100,7 @@ def build(verbose: bool = False, jobs: int = 8, incremental: bool = False) -> Pa
         return obj
 
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as pool:
-        objects = list(pool.map(compile_one, sources()))
+        objects = list(pool.map(compile_one, sources(regenerate)))
     resources = {}
     for obj in objects:
         resources.update(json.loads(obj.with_suffix(".resources.json").read_text()))
@@ -163,4 +166,5 @@ def _build_torchcall(verbose: bool) -> None:
 
 
 if __name__ == "__main__":
-    print(build(verbose="-v" in sys.argv[1:], incremental="--incremental" in sys.argv[1:]))
+    print(build(verbose="-v" in sys.argv[1:], incremental="--incremental" in sys.argv[1:],
+                regenerate="--as-generated" not in sys.argv[1:]))
