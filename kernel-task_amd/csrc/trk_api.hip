@@ -3,7 +3,7 @@
 // A plan fixes one operator shape and dtype, the contraction orders its kernels use (each
 // with a section of the packed-core buffer) and a table of kernel variants with the token
 // counts each one serves. Host-only logic: nothing here calls HIP except trk_pack,
-// trk_forward* and trk_empty_launch.
+// trk_plan_admit, trk_forward* and trk_empty_launch.
 #include <dlfcn.h>
 
 #include <algorithm>
@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <new>
 
 #include "trk_internal.h"
@@ -392,16 +393,27 @@ int trk_plan_admit(trk_plan *plan, const void *packed, void *stream) {
     if (p.dtype != TRK_DTYPE_F16 || p.admitted < 0) return TRK_OK;
     for (int i = 0; i < p.nchains; ++i) {
         if (!p.chains[i].join) continue;
-        unsigned uneven = 1;
-        const char *verdict = static_cast<const char *>(packed) + p.chains[i].offF + 4 * kJoinUneven;
-        int st = check_hip(hipMemcpyAsync(&uneven, verdict, sizeof(uneven), hipMemcpyDeviceToHost,
-                                          static_cast<hipStream_t>(stream)),
-                           "trk_plan_admit: copy");
+        // one word of pinned memory for the process, held by one call at a time; never freed (a call
+        // may come while static objects are destroyed)
+        static std::mutex held;
+        static unsigned *uneven = nullptr;
+        std::lock_guard<std::mutex> lock(held);
+        if (!uneven) {
+            void *word = nullptr;
+            const int st = check_hip(hipHostMalloc(&word, sizeof(*uneven),
+                                         hipHostMallocPortable | hipHostMallocMapped),
+                           "trk_plan_admit: pinned word");
+            if (st != TRK_OK) return st;
+            uneven = static_cast<unsigned *>(word);
+        }
+        *uneven = 1;
+        int st = launch_join_verdict(static_cast<const char *>(packed) + p.chains[i].offF, uneven,
+                                     static_cast<hipStream_t>(stream));
         if (st == TRK_OK)
             st = check_hip(hipStreamSynchronize(static_cast<hipStream_t>(stream)),
                            "trk_plan_admit: wait");
         if (st != TRK_OK) return st;
-        p.admitted = uneven ? -1 : 1;
+        p.admitted = *uneven ? -1 : 1;
     }
     return TRK_OK;
 }

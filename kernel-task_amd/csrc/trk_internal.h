@@ -114,6 +114,8 @@ constexpr const char *kModuleAbi = "trk_module_abi";
 // kernels and their launchers
 int launch_pack(const Plan &plan, const void *g1, const void *g2, const void *g3, void *packed,
                 hipStream_t stream);                                   // trk_pack.hip
+// word kJoinUneven of the joined-core section `section` into pinned host memory
+int launch_join_verdict(const void *section, unsigned *host, hipStream_t stream);  // trk_pack.hip
 // generic kernel variant of `chain` whose workgroups own `sg` second-core outputs each
 int generic_configure(const Plan &plan, int chain, int sg, Variant *v);  // trk_generic.hip
 int launch_generic(const Plan &plan, const Variant &v, const void *packed, const void *x,
