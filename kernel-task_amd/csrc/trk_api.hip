@@ -136,9 +136,9 @@ int plan_join_chain(Plan *p) {
     c.join = 1;
     c.ownF = c.ownS = c.ownL = 0;
     const size_t e = size_t(p->elem), R2 = size_t(c.R) * c.R;
-    if (R2 * (1 + 16 * size_t(c.nL) + size_t(c.oF) * c.nF + size_t(c.oS) * c.nS) >> 31) return -1;
+    if (R2 * (16 * size_t(c.nL) + size_t(c.oF) * c.nF + size_t(c.oS) * c.nS) >> 31) return -1;
     c.offF = p->packed_bytes;
-    c.offL = c.offF + kJoinHeader + e * R2;                 // J1: G1's fragments
+    c.offL = c.offF + kJoinHeader;                           // J1: G1's fragments
     c.offS = c.offL + e * R2 * 16 * c.nL;                    // J2, then J3
     p->packed_bytes = align256(c.offS + e * R2 * (size_t(c.oF) * c.nF + size_t(c.oS) * c.nS));
     return p->nchains++;

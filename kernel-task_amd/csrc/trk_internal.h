@@ -99,8 +99,8 @@ int plan_chain(Plan *plan, const int order[3], int sg, int lg, int sfrag);
 // index of the plan's joined-core section, added if new (-1: full)
 int plan_join_chain(Plan *plan);
 // The joined-core section: kJoinHeader bytes whose first float is the factor of the results and
-// whose word kJoinUneven is nonzero for fp16 cores too uneven for one scale each, R^2 zeros, then
-// J1, J2 and J3 (trk_pack.hip).
+// whose word kJoinUneven is nonzero for fp16 cores too uneven for one scale each, then J1, J2 and J3
+// (trk_pack.hip).
 constexpr int kJoinHeader = 256, kJoinUneven = 63;
 
 // Entry points a variant module (a generated table built at prepare time) exports, and the

@@ -85,9 +85,9 @@ struct JoinGeo {
         return worst;
     }
     static constexpr int NH = SJ ? 1 : cdiv(span(), 2);
-    // packed section (trk_pack.hip): header (the output scale), zeros, then
+    // packed section (trk_pack.hip): header (the output scale), then
     // J1[i][K step][lane][8], J2[q][j][b][c], J3[r][k][a][c]
-    static constexpr int oJ1 = kJoinHeader / EB + R2;
+    static constexpr int oJ1 = kJoinHeader / EB;
     static constexpr int oJ2 = oJ1 + nI * KS * FRAG;
     static constexpr int oJ3 = oJ2 + oQ * nJ * R2;
     // LDS, in elements: the workgroup's slices of G2 and G3 (rows of one k 16 bytes past

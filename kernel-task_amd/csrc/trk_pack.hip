@@ -136,7 +136,7 @@ int pack_all(const Plan &plan, const void *const g[3], void *packed, hipStream_t
     return TRK_OK;
 }
 
-// The joined-core section (trk_join_kernel.h): [header][R^2 zeros][J1][J2][J3].
+// The joined-core section (trk_join_kernel.h): [header][J1][J2][J3].
 //   J1[i][step][lane][8] = G1[a,p,i,b] as the formation's B fragments: column p = lane % 16 (zero
 //                          at or past oP), K position 8 g + u of lane group g = lane / 16 being
 //                          (a, b) in the order two results of the join (rows 4 g + u % 4) make a
@@ -276,15 +276,14 @@ __global__ void __launch_bounds__(256) join_pack_kernel(
             exponents[k] = join_exponent(reinterpret_cast<const float *>(out) + 1 + k * kPeaks);
     const int R = a.R, R2 = R * R;
     T *dst = reinterpret_cast<T *>(out + kJoinHeader);
-    const unsigned total = R2 + a.nJ1 + a.nJ2 + a.nJ3;
+    const unsigned total = a.nJ1 + a.nJ2 + a.nJ3;
     if (blockIdx.x == 0 && threadIdx.x == 0)
         *reinterpret_cast<float *>(out) = ldexpf(1.0f, exponents[0] + exponents[1] + exponents[2]);
     for (unsigned d = blockIdx.x * blockDim.x + threadIdx.x; d < total; d += gridDim.x * blockDim.x) {
         float v = 0.0f;
         int core = 0;
-        if (d < unsigned(R2)) {
-        } else if (d < R2 + a.nJ1) {
-            const unsigned e = d - R2;
+        if (d < a.nJ1) {
+            const unsigned e = d;
             const int in = int(e % 512), s = int(e / 512 % (R2 / 32)), i = int(e / 512 / (R2 / 32));
             const int lane = sizeof(T) == 2 ? in / 8 : in % 256 / 4;
             const int u = sizeof(T) == 2 ? in % 8 : in / 256 * 4 + in % 4;
@@ -293,15 +292,15 @@ __global__ void __launch_bounds__(256) join_pack_kernel(
             const int cb = R == 8 ? 4 * (g % 2) + u % 4 : 4 * g + u % 4;
             if (p < a.oP && ca < a.Rc && cb < a.Rc)
                 v = E::to_f32(g1[core_index(ca, p, i, cb, a.oP, a.nI, a.Rc)]);
-        } else if (d < R2 + a.nJ1 + a.nJ2) {
-            const unsigned e = d - R2 - a.nJ1;
+        } else if (d < a.nJ1 + a.nJ2) {
+            const unsigned e = d - a.nJ1;
             const int cc = int(e % R), cb = int(e / R % R), j = int(e / R2 % a.nJ);
             const int q = int(e / R2 / a.nJ);
             core = 1;
             if (cb < a.Rc && cc < a.Rc)
                 v = E::to_f32(g2[core_index(cb, q, j, cc, a.oQ, a.nJ, a.Rc)]);
         } else {
-            const unsigned e = d - R2 - a.nJ1 - a.nJ2;
+            const unsigned e = d - a.nJ1 - a.nJ2;
             const int cc = int(e % R), ca = int(e / R % R), k = int(e / R2 % a.nK);
             const int r = int(e / R2 / a.nK);
             core = 2;
@@ -341,7 +340,7 @@ int pack_join(const Plan &plan, const Chain &c, const void *const g[3], void *pa
                            static_cast<const _Float16 *>(g[0]), static_cast<const _Float16 *>(g[1]),
                            static_cast<const _Float16 *>(g[2]), header, a);
     }
-    const unsigned total = R2 + a.nJ1 + a.nJ2 + a.nJ3;
+    const unsigned total = a.nJ1 + a.nJ2 + a.nJ3;
     hipLaunchKernelGGL(join_pack_kernel<DT>, dim3(std::min(total / 256 + 1, 4096u)), dim3(256), 0,
                        stream, t[0], t[1], t[2], out, a);
     return check_hip(hipGetLastError(), "trk_pack: launch");
