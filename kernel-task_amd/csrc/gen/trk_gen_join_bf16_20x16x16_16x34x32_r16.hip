@@ -1,5 +1,5 @@
 // Generated by kernel-task_amd/factorized_inference/tilegen.py; do not edit.
-// qwen_mlp_gate_up: (20,16,16) -> (16,34,32), rank 16, bf16, chain order (1,2,0); token ranges measured by kernel-task_amd/benchmarks/autotune.py.
+// qwen_mlp_gate_up: (20,16,16) -> (16,34,32), rank 16, bf16, chain order (1,2,0); token ranges measured by kernel-task_amd/benchmarks/autotune.py --joined.
 #include "trk_join_kernel.h"
 
 namespace trk {

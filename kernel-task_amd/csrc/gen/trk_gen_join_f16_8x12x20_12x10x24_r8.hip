@@ -1,5 +1,5 @@
 // Generated by kernel-task_amd/factorized_inference/tilegen.py; do not edit.
-// r8: (8,12,20) -> (12,10,24), rank 8, f16, chain order (1,2,0); token ranges measured by kernel-task_amd/benchmarks/autotune.py.
+// r8: (8,12,20) -> (12,10,24), rank 8, f16, chain order (1,2,0); token ranges measured by kernel-task_amd/benchmarks/autotune.py --joined, for cores that trk_plan_admit finds even.
 #include "trk_join_kernel.h"
 
 namespace trk {

@@ -13,9 +13,11 @@
 // No weight is ever stored: a wave forms 32 x 16 values at a time, in the registers that its
 // next MFMAs read, and drops them.
 //
-// Everything between the core loads and y stays in registers. In a 16x16 MFMA a lane holds
-// four consecutive rows of one result column; as an operand it holds eight K positions of one
-// row or column. So a result whose rows are the next contraction's index becomes that
+// Everything between the core loads and y is held in registers. (Two kinds of kernels spill some:
+// 1920 -> 2880 R16 fp16 with 256 tokens a workgroup, 19 VGPRs, and most fused pairs, which keep the
+// gate's results through the second pass, up to 189; their times chose them all the same.) In a
+// 16x16 MFMA a lane holds four consecutive rows of one result column; as an operand it holds eight
+// K positions of one row or column. So a result whose rows are the next contraction's index becomes that
 // contraction's operand without leaving the lane, two 16-row results making one 32-wide K
 // step (rounded to the plan's type on the way, as U and V are in the chains), provided the
 // other operand orders its K the same way:

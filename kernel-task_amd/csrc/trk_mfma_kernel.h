@@ -174,8 +174,9 @@ struct KCfg {
                              // run it (s_setprio), so that they finish before the waves with
                              // whole row tiles instead of after them, waiting on LDS alone
     int JN;                  // 1: a joined-core tile (trk_join_kernel.h): TT tokens x (FC x SC)
-                             // pairs of output digits x all LC digits of G1, IC input digits
-                             // of G1 in LDS at a time, KS3 waves splitting the features
+                             // pairs of output digits x all LC digits of G1, steps of IC = 1
+                             // input digit of G1 (two steps in LDS), KS3 waves splitting the
+                             // features
 };
 
 // K orders of the packed second- and last-core sections a variant reads (its chain's layout):

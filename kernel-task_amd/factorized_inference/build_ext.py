@@ -41,8 +41,8 @@ HIPCC_FLAGS = [
 
 
 def file_flags(src: Path) -> list[str]:
-    """HIPCC_FLAGS of one source. The joined-core tiles (csrc/trk_join_kernel.h) hold up to 400
-    registers a lane: with accumulators allowed in the accumulation half of the register file
+    """HIPCC_FLAGS of one source. The joined-core tiles (csrc/trk_join_kernel.h) hold up to all
+    512 registers a lane: with accumulators allowed in the accumulation half of the register file
     they need no copies between the halves, where the VGPR form of the MFMAs copies its operands
     there and back (measured at 14336 -> 4096 R16, T=2048, 256 tokens a workgroup: 421 us against
     866). The other kernels fit the VGPR half."""

@@ -109,8 +109,8 @@ class Tile:
     TP: int = 0    # 1: the tail waves of a pair-and-tail stage 2 hold the issue priority while
     #                they run it (KCfg::TP; tiles with tail waves only)
     JN: int = 0    # 1: a joined-core tile (csrc/trk_join_kernel.h): TT tokens x (FC x SC) pairs
-    #                of second- and third-core output digits x all of the first core's, IC input
-    #                digits of the first core in LDS at a time, KS3 waves splitting the features
+    #                of second- and third-core output digits x all LC of the first core's, steps of
+    #                IC = 1 of its input digits (two steps in LDS), KS3 waves splitting the features
 
     def args(self) -> str:
         """Arguments of tile(shape, ...) in the variant tables."""
@@ -279,8 +279,9 @@ def join_geometry(shape: ShapeDecl, order: tuple, t: Tile) -> dict:
     x_step = t.KS3 * rup(t.TT, max(rows, 16)) * 32 + (0 if shared else skew + vpe)
     lds = max(eb * (slices + R * R + 2 * ks * 512 + 2 * x_step),
               min(mt, 4) * 16 * (pairs * 16 + 4) * 4 if shared else t.NW * nq * mt * 1024)
-    # registers of the arrays: accumulators, the joined slice and G1's fragments, x read from LDS,
-    # two steps of it in flight, a formed tile, and addresses
+    # registers of the plain kernel's arrays: accumulators, the joined slice and G1's fragments, x
+    # read from LDS, two steps of it in flight, a formed tile, and addresses. The fused pair also
+    # keeps the gate's results and may spill: it is chosen by its time (autotune.py --joined).
     vgprs = (nq * mt * 4 + (nq * 2 + 1) * ks * 2 * eb + mt * 2 * eb + 9 * cdiv(t.TT, rows)
              + nq * (8 + 2 * eb) + 28)
     g = {"LDS_BYTES": lds, "NBLK": cdiv(q, t.FC) * cdiv(r, t.SC), "TAIL": False,
@@ -890,6 +891,8 @@ def emit(shape: ShapeDecl, tuned: dict | None = None, all_candidates: bool = Fal
     orders = sorted({r[1] for r in rows}, key=lambda od: (od != choose_order(shape), od))
     i, o = shape.ins, shape.outs
     tuned_note = ("token ranges measured by kernel-task_amd/benchmarks/autotune.py"
+                  + (" --joined" + (", for cores that trk_plan_admit finds even"
+                                    if shape.dtype == "f16" else "") if join else "")
                   if tuned.get(shape.key) and not all_candidates
                   else "every candidate, token ranges by rule (not tuned)")
     lines = [

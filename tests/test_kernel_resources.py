@@ -37,3 +37,22 @@ def test_no_stack_objects_in_mfma_kernels(resources):
 def test_lds_within_160_kb(resources):
     for n, r in resources.items():
         assert int(r["LDS Size"]) <= 160 * 1024, n
+
+
+def test_no_stack_objects_in_joined_kernels(resources):
+    # the joined-core kernels, the fused pairs among them: scratch is for spilled registers alone
+    joined = {n: r for n, r in resources.items() if "ring3_join" in n}
+    assert any("ring3_join_kernel" in n for n in joined)
+    assert any("ring3_join_pair_kernel" in n for n in joined)
+    bad = [n for n, r in joined.items()
+           if int(r["ScratchSize"]) > 0 and int(r.get("VGPRs Spill", "0")) == 0]
+    assert not bad, f"{len(bad)} joined kernels hold register arrays in scratch, e.g. {bad[:2]}"
+
+
+def test_only_one_plain_joined_tile_spills(resources):
+    # 1920 -> 2880 R16 fp16 with 256 tokens and 8 output pairs a workgroup (KCfg fields: dtype, order,
+    # modes, rank, TT, FC, SC); the pairs, which keep the gate's results as well, mostly do
+    spills = [n for n, r in resources.items()
+              if "ring3_join_kernel" in n and int(r.get("VGPRs Spill", "0")) > 0]
+    tile = "KCfgELi0ELi1ELi2ELi0ELi8ELi12ELi20ELi12ELi10ELi24ELi16ELi256ELi1ELi8E"
+    assert spills and all(tile in n for n in spills), spills

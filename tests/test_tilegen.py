@@ -284,3 +284,22 @@ def test_candidates_with_one_name_keep_both_tiles():
     assert tilegen.add_candidate(cands, "w~t1", order, t1) is None
     assert tilegen.add_candidate(cands, "w~t1", (0, 1, 2), t1) == "w~t1#3"
     assert cands == {"w~t1": (order, t1), "w~t1#2": (order, t2), "w~t1#3": ((0, 1, 2), t1)}
+
+
+@pytest.mark.parametrize("change,why", [
+    ({}, ""),
+    ({"TT": 40}, "tiles of 16"),
+    ({"IC": 2}, "one first-core digit"),
+    ({"LC": 12}, "16 columns"),
+    ({"KS3": 3}, "divide the waves"),
+    ({"KS3": 1}, "split over the waves"),          # 2 pairs, 8 waves
+    ({"FC": 3, "SC": 4, "KS3": 4}, "whole rows"),  # 6 pairs a wave in rows of 4
+    ({"KS3": 8, "TT": 256}, "LDS"),
+    ({"TT": 64, "FC": 4}, "registers"),            # the joined slices of 4 pairs a wave
+    ({"NACC": 2}, "two waves"),
+])
+def test_planted_joined_tile_mistakes_are_rejected(change, why):
+    # 14336 -> 4096 R16: 128 tokens x two pairs a workgroup, four waves to the features, two to a pair
+    tile = replace(tilegen.Tile(128, 1, 2, 16, 1, 4, 1, NW=8, JN=1), **change)
+    reject = tilegen.geometry(HAND[3], tilegen.JOIN_ORDER, tile)["reject"]
+    assert why in reject and bool(why) == bool(reject), reject
