@@ -5,6 +5,8 @@ the 16 columns, zero-padded ranks, epilogues at every alignment of y, cores far 
 launch. Against the float64 oracle, on the first and last rows (token rows are independent)."""
 from __future__ import annotations
 
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 import torch
@@ -121,7 +123,7 @@ def test_fp16_cores_far_from_one(scales):
         assert np.linalg.norm(y - expected) <= 2.0 ** -10 * norm, info["name"]
 
 
-@pytest.mark.parametrize("rank", [8, 16])
+@pytest.mark.parametrize("rank", [8, 12, 16])  # 12: zero-padded to 16, the padding not looked at
 @pytest.mark.parametrize("name", jm.CASES)
 def test_fp16_calls_are_exact_for_uneven_cores(name, rank):
     # joined tiles form products of two and three cores in fp16: cores whose slices differ in size
@@ -150,6 +152,20 @@ def test_swiglu_pair_of_joined_tiles():
         x = torch.randn(t, spec.in_features, device="cuda", dtype=dtype,
                         generator=torch.Generator(device="cuda").manual_seed(t))
         assert torch.equal(forward_swiglu(gate, up, x), up.forward_silu_mul(x, gate.accumulate(x)))
+
+
+def test_operators_prepared_by_several_threads_are_admitted_each_by_its_cores():
+    names = ["plain", "entry_100", "laplace", "input_100"] * 4
+    made = [[c.cuda() for c in jm.make(n, 8, 1)[1]] for n in names]
+    torch.cuda.synchronize()
+
+    def prepare(cores):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            return prepare_optimized(cores, TRSpec(jm.INS, jm.OUTS, 8))
+
+    with ThreadPoolExecutor(4) as pool:
+        for name, run in zip(names, pool.map(prepare, made)):
+            assert ("join" in run.selected(201)["name"]) == (name in ("plain", "laplace")), name
 
 
 @pytest.mark.parametrize("shape,rank", [("llama_up", 8), ("gate_up", 8), ("gate_up", 16)])
